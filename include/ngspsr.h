@@ -387,6 +387,28 @@ int ngs_pcg_solve_packed(const int32_t *runs, const float *pvals, const int64_t 
                          const float *b, float *x, int64_t M, double tol, int32_t max_iter, int32_t chunk,
                          void *workspace, ngs_stream_t s, int32_t *iters, double *rel_resid);
 
+/* Filtered preconditioner of ngs_pcg_solve_packed_filtered (no reference counterpart): D^-1/2 P D^-1/2
+ * in place of D^-1, P a 27-point filter on the level's voxels. words: ngs_level_filter_words of the
+ * level; weights: P_ij for voxels whose offset has 1, 2 and 3 non-zero components in {-1, 0, 1} (1 for a
+ * voxel itself). P is positive definite on every voxel set when its symbol
+ * 1 + 2 w0 (a+b+c) + 4 w1 (ab+ac+bc) + 8 w2 abc is positive at the 8 corners a, b, c = +-1 (the symbol is
+ * linear in each cosine); checked. */
+typedef struct ngs_pcg_filter {
+    const int32_t *words;
+    float weights[3];
+    float pad_;
+} ngs_pcg_filter;
+/* Filter words of a level: 9 plane-major int32 per row (plane stride M rounded up to 64), plane
+ * 3 (dx + 1) + (dy + 1): rank of the first present voxel of (dx, dy, -1 .. 1) in the low 29 bits, the
+ * presence mask of dz = -1, 0, 1 in the top 3. */
+int ngs_level_filter_words(ngs_level level, int32_t *words, ngs_stream_t s);
+/* ngs_pcg_solve_packed with the filtered preconditioner: the same stop rule (||r|| <= tol ||b||,
+ * recurrence residual) after fewer iterations. */
+int ngs_pcg_solve_packed_filtered(const int32_t *runs, const float *pvals, const int64_t *soff, const float *inv_diag,
+                                  ngs_pcg_filter filter, const float *b, float *x, int64_t M, double tol,
+                                  int32_t max_iter, int32_t chunk, void *workspace, ngs_stream_t s, int32_t *iters,
+                                  double *rel_resid);
+
 /* ngs_pcg_solve on the stencil form of the system (same iteration, same stop rule; the SpMV is the
  * point pass + row pass of ngs_stencil_apply). */
 int ngs_pcg_solve_stencil(ngs_stencil op, const float *inv_diag, const float *b, float *x, double tol,
@@ -420,6 +442,11 @@ int ngs_pcg_batch_prepare_runs(const int32_t *runs, const float *rvals, const fl
 int ngs_pcg_batch_prepare_packed(const int32_t *runs, const float *pvals, const int64_t *soff, const float *inv_diag,
                                  const float *b, float *x, int64_t M, double tol, int32_t max_iter, void *workspace,
                                  int32_t blk0, int32_t nblk, void *entry, ngs_stream_t s);
+/* The same with the filtered preconditioner (ngs_pcg_solve_packed_filtered); needs flag bit 4. */
+int ngs_pcg_batch_prepare_packed_filtered(const int32_t *runs, const float *pvals, const int64_t *soff,
+                                          const float *inv_diag, ngs_pcg_filter filter, const float *b, float *x,
+                                          int64_t M, double tol, int32_t max_iter, void *workspace, int32_t blk0,
+                                          int32_t nblk, void *entry, ngs_stream_t s);
 /* The same as ngs_pcg_batch_prepare for a system in stencil form. */
 int ngs_pcg_batch_prepare_stencil(ngs_stencil op, const float *inv_diag, const float *b, float *x, double tol,
                                   int32_t max_iter, void *workspace, int32_t blk0, int32_t nblk, void *entry,
@@ -427,7 +454,8 @@ int ngs_pcg_batch_prepare_stencil(ngs_stencil op, const float *inv_diag, const f
 /* `iters` (even) iterations of every active system in one launch per kernel (graph-replayed when
  * use_graph). flags: bit 0 the table may hold stencil systems (adds their point and row passes),
  * bit 1 it may hold run-form systems (adds their SpMV), bit 2 it holds no CSR systems (skips
- * that SpMV), bit 3 it may hold packed-form systems (adds their SpMV). */
+ * that SpMV), bit 3 it may hold packed-form systems (adds their SpMV), bit 4 some of those are filtered
+ * (adds the filter step). */
 int ngs_pcg_batch_iterate(const void *table, const int32_t *blk2sys, int32_t total_blocks, int32_t iters,
                           int32_t use_graph, int32_t flags, ngs_stream_t s);
 /* (iter, done) of each system of the host copy of the table into states (2 nsys int32, host),

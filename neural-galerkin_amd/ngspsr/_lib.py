@@ -43,6 +43,10 @@ class HashTable(ctypes.Structure):
                 ("pad_", c_int32)]
 
 
+class PcgFilter(ctypes.Structure):
+    _fields_ = [("words", c_void_p), ("weights", c_float * 3), ("pad_", c_float)]
+
+
 P = c_void_p
 _SIGNATURES = {
     "ngs_last_error": ([], ctypes.c_char_p),
@@ -135,6 +139,11 @@ _SIGNATURES = {
                               ctypes.POINTER(c_double)], c_int32),
     "ngs_pcg_batch_prepare_packed": ([P, P, P, P, P, P, c_int64, c_double, c_int32, P, c_int32, c_int32, P, P],
                                      c_int32),
+    "ngs_level_filter_words": ([Level, P, P], c_int32),
+    "ngs_pcg_solve_packed_filtered": ([P, P, P, P, PcgFilter, P, P, c_int64, c_double, c_int32, c_int32, P, P,
+                                       ctypes.POINTER(c_int32), ctypes.POINTER(c_double)], c_int32),
+    "ngs_pcg_batch_prepare_packed_filtered": ([P, P, P, P, PcgFilter, P, P, c_int64, c_double, c_int32, P, c_int32,
+                                               c_int32, P, P], c_int32),
     "ngs_residual_f64_packed": ([P, P, P, P, P, P, c_int64, P, P, P], c_int32),
     "ngs_stencil_pass": ([Stencil, P, P, c_int32, P], c_int32),
     "ngs_stencil_row_counts": ([Level, P, P], c_int32),

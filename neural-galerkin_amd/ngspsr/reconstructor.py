@@ -219,7 +219,9 @@ class Reconstructor:
                 pvals = torch.empty(max(nvals, 1), dtype=torch.float32, device=dev)
                 call("ngs_lhs_assemble_packed", lv, pb, ptr(coarse), float(sf), float(delta), ptr(runs), ptr(pvals),
                      ptr(soff), ptr(inv_diag), ptr(rhs), stream())
-                return _solver.RunSystem.from_packed(runs, pvals, soff, inv_diag)
+                system = _solver.RunSystem.from_packed(runs, pvals, soff, inv_diag)
+                system.set_level(tree.grids[d], tree.strides[d], self._screening_strength(d, bins, sf))
+                return system
             if _solver.RunSystem.PACKED:
                 # the slot values only feed the packing: a thread scratch buffer, reused level to level
                 rvals = Scratch.get(125 * P * 4, dev, slot=7)[:125 * P * 4].view(torch.float32).view(125, P)
@@ -227,7 +229,9 @@ class Reconstructor:
                 rvals = torch.empty((125, P), dtype=torch.float32, device=dev)
             call("ngs_lhs_assemble_runs", lv, pb, ptr(coarse), float(sf), float(delta), ptr(runs),
                  ptr(rvals), ptr(inv_diag), ptr(rhs), stream())
-            return _solver.RunSystem(runs, rvals, inv_diag, layout=layout)
+            system = _solver.RunSystem(runs, rvals, inv_diag, layout=layout)
+            system.set_level(tree.grids[d], tree.strides[d], self._screening_strength(d, bins, sf))
+            return system
         if form != "csr":
             raise ValueError(f"unknown operator form {form!r}")
         row_nnz = torch.empty(M, dtype=torch.int32, device=dev)
@@ -241,6 +245,18 @@ class Reconstructor:
         call("ngs_lhs_assemble", lv, pb, ptr(coarse), float(sf), float(delta), ptr(rowptr), ptr(cols),
              ptr(vals), ptr(inv_diag), ptr(rhs), stream())
         return _solver.CSRSystem(rowptr, cols, vals, inv_diag)
+
+    def _screening_strength(self, d, bins, sf):
+        """Mean diagonal of the screening term over that of the stiffness, from the sizes: a point adds
+        alpha sf prod_axes int B^2 = alpha sf 2.2^3 to the diagonals in all, a row's stiffness is
+        3 int B'^2 (int B^2)^2 s = 58.08 s. Per-point weights stand in the middle of the filters' range
+        (their values are on the device), 0 without points."""
+        if not bins.n:
+            return 0.0
+        if bins.alpha is not None:
+            return 0.2
+        M = self.hash_tree.level(d).M
+        return sf * bins.alpha_scalar * bins.n * 2.2 ** 3 / (M * 58.08 * self.hash_tree.strides[d])
 
     def _add_field_at_points(self, d, sol, xyz, bins, out):
         """out += level d's field at the screening points (ngs_eval_field's values bit for bit), read

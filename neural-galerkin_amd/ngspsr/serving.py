@@ -26,10 +26,12 @@ from .reconstructor import Reconstructor
 
 
 class _Job:
-    __slots__ = ("system", "b", "x", "ws", "tol", "max_iter", "done", "iters", "status", "ready", "nblk", "t0")
+    __slots__ = ("system", "b", "x", "ws", "tol", "max_iter", "done", "iters", "status", "ready", "nblk", "t0",
+                 "filt")
 
-    def __init__(self, system, b, tol, max_iter):
+    def __init__(self, system, b, tol, max_iter, filt=None):
         self.system = system
+        self.filt = filt
         self.b = b.float().contiguous()
         self.x = torch.empty(system.M, dtype=torch.float32, device=system.device)
         self.ws = torch.empty(lib().ngs_pcg_workspace_bytes(system.M), dtype=torch.uint8, device=system.device)
@@ -87,11 +89,11 @@ class BatchedPCG:
         self.thread = threading.Thread(target=self._run, name="ngspsr-pcg-pool", daemon=True)
         self.thread.start()
 
-    def solve(self, system, b, tol=1e-6, max_iter=100000):
-        """Blocking solve through the pool (callable from any worker thread)."""
+    def solve(self, system, b, tol=1e-6, max_iter=100000, filt=None):
+        """Blocking solve through the pool (callable from any worker thread); filt as in solver.pcg."""
         if self._err is not None:
             raise self._err
-        job = _Job(system, b, tol, max_iter)
+        job = _Job(system, b, tol, max_iter, filt)
         self.pending.put(job)
         self._wake.set()
         while not job.done.wait(0.5):
@@ -139,6 +141,11 @@ class BatchedPCG:
                 call("ngs_pcg_batch_prepare_stencil", s.struct(), ptr(s.inv_diag), ptr(job.b), ptr(job.x),
                      float(job.tol), int(job.max_iter), ptr(job.ws), 0, job.nblk, entry.data_ptr(),
                      self.stream.cuda_stream)
+            elif job.filt is not None:
+                pvals, soff = s._packed
+                call("ngs_pcg_batch_prepare_packed_filtered", ptr(s.runs), ptr(pvals), ptr(soff), ptr(s.inv_diag),
+                     job.filt.struct, ptr(job.b), ptr(job.x), s.M, float(job.tol), int(job.max_iter), ptr(job.ws), 0,
+                     job.nblk, entry.data_ptr(), self.stream.cuda_stream)
             elif isinstance(s, _solver.RunSystem) and s.is_packed:
                 pvals, soff = s._packed
                 call("ngs_pcg_batch_prepare_packed", ptr(s.runs), ptr(pvals), ptr(soff), ptr(s.inv_diag), ptr(job.b),
@@ -174,6 +181,8 @@ class BatchedPCG:
                         self.dev_map.copy_(self.host_map, non_blocking=True)
                         self._dirty = False
                     flags = launch_flags(j.system for j in self.active)
+                    if any(j.filt is not None for j in self.active):
+                        flags |= 16
                     call("ngs_pcg_batch_iterate", ptr(self.dev_table), ptr(self.dev_map), self.cap, self.chunk,
                          int(self.use_graph), flags, self.stream.cuda_stream)
                     self.launches += 1
@@ -283,9 +292,10 @@ class ReconstructionServer:
         nb = math.sqrt(bb)
         rel = math.sqrt(rr) / nb if nb > 0 else 0.0
         info = _solver.SolveInfo()
+        filt = _solver.system_filter(system) if rel > self.tol else None
         while rel > self.tol and info.outer < 20:
-            inner_tol = _solver.inner_tolerance(self.tol, self.inner_tol, info.outer)
-            e, inner = self.pool.solve(system, r64.float(), tol=inner_tol)
+            inner_tol = _solver.inner_tolerance(self.tol, self.inner_tol, info.outer, filt is not None)
+            e, inner = self.pool.solve(system, r64.float(), tol=inner_tol, filt=filt)
             x64 += e.double()
             info.iters += inner.iters
             info.outer += 1

@@ -15,7 +15,8 @@ Solver strings keep the reference's mini-language, "pcg@tol=1e-6@maxiter=1000@re
            singularity, as cuSOLVER reports it.
   refine   FP64 iterative refinement around FP32 inner PCG solves (no reference counterpart):
            r = b - A x in FP64, inner solve A e = r to inner_tol, x += e in FP64, until
-           ||b - A x|| / ||b|| <= tol.
+           ||b - A x|| / ||b|| <= tol. The inner solves of packed run-form levels with screening take the
+           filtered preconditioner (RunSystem.filter): "pcg" keeps the reference's Jacobi iteration.
 """
 import ast
 import ctypes
@@ -87,6 +88,13 @@ class CSRSystem:
         return a
 
 
+class Filter:
+    """A filtered preconditioner: the words tensor (kept alive here) and the struct the kernels take."""
+
+    def __init__(self, words, struct):
+        self.words, self.struct = words, struct
+
+
 class RunSystem:
     """Assembled level system in run form (ngs_lhs_assemble_runs): for each row and each of the 25
     bitmap columns (dx, dy) of its 5x5x5 neighbourhood, one run word (first column | count << 28)
@@ -114,6 +122,7 @@ class RunSystem:
         assert runs.shape == (25, self.plane_stride(self.M)) and rvals.shape == (125, self.plane_stride(self.M))
         self._rvals = rvals
         self._packed = None
+        self.level_grid = None
         if (self.PACKED if packed is None else packed) and self.M:
             self._pack(rvals, layout)
             self._rvals = None
@@ -128,7 +137,42 @@ class RunSystem:
         assert runs.shape == (25, cls.plane_stride(self.M)) and soff.shape == ((self.M + 63) // 64 + 1,)
         self._rvals = None
         self._packed = (pvals, soff)
+        self.level_grid = None
         return self
+
+    def set_level(self, grid, stride: int, screening: float):
+        """The level's SparseGrid (rows in rank order) and stride, and the strength of its screening term
+        beside the stiffness (mean diagonal of one over the other; 0 without screening): what filter()
+        needs. Held by the system, since the filter's words are made from the grid."""
+        self.level_grid, self.level_stride, self.screening = grid, int(stride), float(screening)
+
+    # P's weights at offsets with 1, 2, 3 non-zero components, by the screening strength up to which they
+    # hold. A stiffness-dominated matrix wants faces damped less than edges and corners lifted; the more
+    # the mass-like screening term dominates, the nearer the best P comes to the inverse mass stencil
+    # (1, -a)^3. Iterations to 1e-7 on levels of five scenes, Jacobi and the four rows:
+    #   strength 0.02: 30 -> 19 22 31 36    0.22: 39 -> 19 17 18 20    0.53: 58 -> 27 23 22 21
+    #   1.5: 66 -> 34 29 26 25              5.9: 106 -> 55 48 42 39
+    FILTERS = ((0.05, (-0.18, 0.06, -0.02)), (0.35, (-0.22, 0.07, -0.02)), (1.0, (-0.23, 0.23 ** 2, -0.23 ** 3)),
+               (float("inf"), (-0.26, 0.26 ** 2, -0.26 ** 3)))
+
+    def filter(self):
+        """The filtered preconditioner of this system for pcg (its words tensor and the kernels' struct),
+        or None: unknown level, unpacked values, or no screening (there Jacobi needs as few iterations:
+        32 against 38 on a 11k-row level of noisy ellipsoids)."""
+        if self._packed is None or self.level_grid is None or not self.screening > 0 or self.M == 0:
+            return None
+        g = self.level_grid
+        lv = _lib.Level()
+        lv.grid = g.struct()
+        lv.coords = g.coords.data_ptr()
+        lv.M = self.M
+        lv.stride = self.level_stride
+        words = torch.empty((9, self.plane_stride(self.M)), dtype=torch.int32, device=self.device)
+        call("ngs_level_filter_words", lv, ptr(words), stream())
+        f = _lib.PcgFilter()
+        f.words = words.data_ptr()
+        f.weights[:] = next(w for top, w in self.FILTERS if self.screening <= top)
+        return Filter(words, f)
 
     def _pack(self, rvals, layout=None):
         nsl = (self.M + 63) // 64
@@ -362,8 +406,9 @@ class SolveInfo:
                 f"true_rel_resid={self.true_rel_resid})")
 
 
-def pcg(system, b, tol=1e-5, maxiter=-1, chunk=32, x_out=None, raise_on_cap=True):
-    """FP32 Jacobi-PCG from x = 0. Returns (x, SolveInfo)."""
+def pcg(system, b, tol=1e-5, maxiter=-1, chunk=32, x_out=None, raise_on_cap=True, filt=None):
+    """FP32 PCG from x = 0: Jacobi, or with filt (RunSystem.filter()) the filtered preconditioner.
+    Returns (x, SolveInfo)."""
     M = system.M
     x = x_out if x_out is not None else torch.empty(M, dtype=torch.float32, device=system.device)
     if M == 0:
@@ -377,7 +422,13 @@ def pcg(system, b, tol=1e-5, maxiter=-1, chunk=32, x_out=None, raise_on_cap=True
                                          int(maxiter), int(chunk), ptr(ws), stream(), ctypes.byref(it),
                                          ctypes.byref(rr))
     elif isinstance(system, RunSystem):
-        if system.is_packed:
+        if filt is not None:
+            pvals, soff = system._packed
+            st = lib().ngs_pcg_solve_packed_filtered(ptr(system.runs), ptr(pvals), ptr(soff), ptr(system.inv_diag),
+                                                     filt.struct, ptr(b), ptr(x), M, float(tol), int(maxiter),
+                                                     int(chunk), ptr(ws), stream(), ctypes.byref(it),
+                                                     ctypes.byref(rr))
+        elif system.is_packed:
             pvals, soff = system._packed
             st = lib().ngs_pcg_solve_packed(ptr(system.runs), ptr(pvals), ptr(soff), ptr(system.inv_diag), ptr(b),
                                             ptr(x), M, float(tol), int(maxiter), int(chunk), ptr(ws), stream(),
@@ -398,13 +449,24 @@ def pcg(system, b, tol=1e-5, maxiter=-1, chunk=32, x_out=None, raise_on_cap=True
 FP32_REACH = 1e-6  # relative residual an FP32 Jacobi-PCG reaches on these systems before it stagnates
 
 
-def inner_tolerance(tol, inner_tol, outer):
+FILTER_CHUNK = 8  # iterations per launch sequence of a filtered solve (11-25 iterations in all, against
+#                   Jacobi's 26-60): one host read per sequence against up to 7 empty iterations
+
+
+def system_filter(system):
+    """The system's filtered preconditioner for the inner solves of iterative refinement, or None."""
+    return system.filter() if isinstance(system, RunSystem) else None
+
+
+def inner_tolerance(tol, inner_tol, outer, filtered=False):
     """Relative tolerance of an inner FP32 solve of iterative refinement. Targets the FP32 solver
     reaches on its own (tol >= 1e-6) are aimed at directly by the first inner solve, to half the
     target so that its FP32 rounding still lands below it, and verified in FP64: one FP32 solve and
-    one FP64 residual. Tighter targets take inner_tol per step (each step gains that factor)."""
+    one FP64 residual. Tighter targets take inner_tol per step (each step gains that factor). A filtered
+    solve gains nearly a factor of two per iteration: it goes to 0.3 of the target, so that where it stops
+    inside that last factor leaves no larger an error than Jacobi's smaller steps did."""
     if outer == 0 and tol >= FP32_REACH:
-        return 0.5 * tol
+        return (0.3 if filtered else 0.5) * tol
     return inner_tol
 
 
@@ -419,9 +481,12 @@ def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, ch
     r64, rr, bb = system.residual_f64(b64, None)  # x = 0: r = b without a matrix pass
     nb = bb ** 0.5
     rel = (rr ** 0.5) / nb if nb > 0 else 0.0
+    filt = system_filter(system) if rel > tol else None
+    if filt is not None:
+        chunk = min(chunk, FILTER_CHUNK)
     while rel > tol and info.outer < max_outer:
-        e, inner = pcg(system, r64.float(), tol=inner_tolerance(tol, inner_tol, info.outer), maxiter=maxiter,
-                       chunk=chunk, raise_on_cap=False)
+        e, inner = pcg(system, r64.float(), tol=inner_tolerance(tol, inner_tol, info.outer, filt is not None),
+                       maxiter=maxiter, chunk=chunk, raise_on_cap=False, filt=filt)
         x64 += e.double()
         info.iters += inner.iters
         info.outer += 1
