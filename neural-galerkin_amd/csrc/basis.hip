@@ -3,6 +3,8 @@
 // backward passes.
 #include "common.h"
 
+#include <algorithm>
+
 namespace ngs {
 
 // p[n, v] = sum_si sum_ti s[n, 3 si + v] t[n, 3 ti + v] ff[si][ti][rel[n, v]], q likewise with dd.
@@ -121,56 +123,106 @@ __global__ void __launch_bounds__(256) ddi_forward_lds_kernel(const float* __res
     }
 }
 
-// Forward with the coefficient rows of 256 consecutive pairs also staged in LDS: the rows are read
-// from global memory as one contiguous, coalesced range per tile (a pair's row is 12 C bytes, so
-// direct per-thread row reads touch a different cache line per lane). Same arithmetic and order.
-constexpr int DDI_TILE = 256;
+// Both directions for NC <= 16 components with everything staged in LDS. A pair's coefficient row is
+// 12 NC bytes, so direct per-thread row reads (and the backward's row writes) touch another cache line
+// per lane: a block copies the rows of 64 consecutive pairs as contiguous ranges, 16 bytes per lane where
+// the arrays are aligned, and the backward's gradients go out the same way, from the LDS slots of the
+// coefficients they replace. One thread per (pair, axis) k = 3 pair + axis: the offsets, the incoming
+// gradients and the forward's results are then contiguous over the lanes too, and the 2 NC coefficients
+// of an axis fit in registers, with every loop over them unrolled. 64 pairs are 192 threads and
+// 1536 NC bytes of LDS beside the tables, so at 7 components the wave slots limit the residency, not the
+// LDS. Arithmetic and
+// summation order are those of the kernels above. 2M pairs of 7 components, forward and backward: 249 and
+// 975 us with a thread per pair (the forward's rows staged, the backward's not).
+constexpr int DDI_PAIRS = 64;
+constexpr int DDI_THREADS = 3 * DDI_PAIRS;
 
-__global__ void __launch_bounds__(DDI_TILE) ddi_forward_tiled_kernel(
-    const float* __restrict__ s, const float* __restrict__ t, const int64_t* __restrict__ rel, int64_t n, int nc,
-    const float* __restrict__ ff, const float* __restrict__ dd, int L, float* __restrict__ p, float* __restrict__ q) {
+__device__ __forceinline__ void ddi_copy(float* __restrict__ dst, const float* __restrict__ src, int n, bool vec) {
+    if (vec && n % 4 == 0) {
+        for (int k = threadIdx.x; k < n / 4; k += DDI_THREADS)
+            reinterpret_cast<float4*>(dst)[k] = reinterpret_cast<const float4*>(src)[k];
+    } else {
+        for (int k = threadIdx.x; k < n; k += DDI_THREADS) dst[k] = src[k];
+    }
+}
+
+template <int NC, bool BWD>
+__global__ void __launch_bounds__(DDI_THREADS) ddi_tile_kernel(const float* __restrict__ s, const float* __restrict__ t,
+                                                               const int64_t* __restrict__ rel, int64_t n,
+                                                               const float* __restrict__ ff,
+                                                               const float* __restrict__ dd, int L, bool vec,
+                                                               const float* __restrict__ gp,
+                                                               const float* __restrict__ gq, float* __restrict__ o1,
+                                                               float* __restrict__ o2) {
 #pragma clang fp contract(off)
-    extern __shared__ float2 tab[];
-    ddi_stage_tables(ff, dd, nc, L, tab);
-    const int w = 3 * nc;
-    float* rs = reinterpret_cast<float*>(tab + (int64_t)L * nc * nc);
-    float* rt = rs + DDI_TILE * w;
-    const int64_t ntiles = (n + DDI_TILE - 1) / DDI_TILE;
+    extern __shared__ float4 ddi_lds[];  // rows of s, rows of t, tables
+    constexpr int W = 3 * NC;
+    float* rs = reinterpret_cast<float*>(ddi_lds);
+    float* rt = rs + DDI_PAIRS * W;
+    float2* tab = reinterpret_cast<float2*>(rt + DDI_PAIRS * W);
+    ddi_stage_tables(ff, dd, NC, L, tab);
+    const int pair = threadIdx.x / 3, v = threadIdx.x - 3 * pair;
+    float* sr = rs + pair * W + v;
+    float* tr = rt + pair * W + v;
+    const int64_t ntiles = (n + DDI_PAIRS - 1) / DDI_PAIRS;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t base = tile * DDI_TILE;
-        const int rows = (int)min((int64_t)DDI_TILE, n - base);
+        const int64_t base = tile * DDI_PAIRS;
+        const int rows = (int)min((int64_t)DDI_PAIRS, n - base);
+        const int64_t k = 3 * base + threadIdx.x;
+        const bool on = pair < rows;
+        // issued with the rows' loads
+        const int64_t r = on ? rel[k] : 0;
+        const float a = BWD && on ? gp[k] : 0.f, b = BWD && on ? gq[k] : 0.f;
         __syncthreads();  // the previous tile's rows are no longer read
-        for (int k = threadIdx.x; k < rows * w; k += DDI_TILE) {
-            rs[k] = s[base * w + k];
-            rt[k] = t[base * w + k];
-        }
+        ddi_copy(rs, s + base * W, rows * W, vec);
+        ddi_copy(rt, t + base * W, rows * W, vec);
         __syncthreads();
-        if ((int)threadIdx.x < rows) {
-            const int64_t i = base + threadIdx.x;
-            const float* sr = rs + threadIdx.x * w;
-            const float* tr = rt + threadIdx.x * w;
+        if (on) {
+            const float2* tb = tab + r * (NC * NC);
+            float sv[NC], tv[NC];
 #pragma unroll
-            for (int v = 0; v < 3; ++v) {
-                const float2* tb = tab + (int64_t)rel[3 * i + v] * nc * nc;
-                float tv[DDI_MAXC];
+            for (int c = 0; c < NC; ++c) {
+                sv[c] = sr[3 * c];
+                tv[c] = tr[3 * c];
+            }
+            if (BWD) {
+                float gacc[NC];
 #pragma unroll
-                for (int ti = 0; ti < DDI_MAXC; ++ti) tv[ti] = ti < nc ? tr[3 * ti + v] : 0.f;
+                for (int c = 0; c < NC; ++c) gacc[c] = 0.f;
+#pragma unroll
+                for (int si = 0; si < NC; ++si) {
+                    float acc = 0.f;
+#pragma unroll
+                    for (int ti = 0; ti < NC; ++ti) {
+                        const float2 w = tb[si * NC + ti];
+                        const float c = a * w.x + b * w.y;
+                        acc += c * tv[ti];
+                        gacc[ti] += c * sv[si];
+                    }
+                    sr[3 * si] = acc;  // this thread's own slots, read above
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c) tr[3 * c] = gacc[c];
+            } else {
                 float pa = 0.f, qa = 0.f;
-                for (int si = 0; si < nc; ++si) {
-                    const float sv = sr[3 * si + v];
 #pragma unroll
-                    for (int ti = 0; ti < DDI_MAXC; ++ti) {
-                        if (ti < nc) {
-                            const float st = sv * tv[ti];
-                            const float2 wt = tb[si * nc + ti];
-                            pa += st * wt.x;
-                            qa += st * wt.y;
-                        }
+                for (int si = 0; si < NC; ++si) {
+#pragma unroll
+                    for (int ti = 0; ti < NC; ++ti) {
+                        const float st = sv[si] * tv[ti];
+                        const float2 w = tb[si * NC + ti];
+                        pa += st * w.x;
+                        qa += st * w.y;
                     }
                 }
-                p[3 * i + v] = pa;
-                q[3 * i + v] = qa;
+                o1[k] = pa;
+                o2[k] = qa;
             }
+        }
+        if (BWD) {
+            __syncthreads();
+            ddi_copy(o1 + base * W, rs, rows * W, vec);
+            ddi_copy(o2 + base * W, rt, rows * W, vec);
         }
     }
 }
@@ -222,7 +274,30 @@ __global__ void __launch_bounds__(256) ddi_backward_lds_kernel(const float* __re
 }
 
 static bool ddi_use_lds(int nc, int L) { return nc <= DDI_MAXC && (int64_t)nc * nc * L * 8 <= DDI_LDS_BYTES; }
-static int64_t ddi_tiled_bytes(int nc, int L) { return (int64_t)nc * nc * L * 8 + 2LL * DDI_TILE * 3 * nc * 4; }
+static int64_t ddi_tile_bytes(int nc, int L) { return (int64_t)nc * nc * L * 8 + 2LL * DDI_PAIRS * 3 * nc * 4; }
+
+// ddi_tile_kernel for nc components; false where its LDS does not fit (the callers' other kernels: tables
+// alone in LDS, or none).
+template <bool BWD, int NC = 1>
+static bool ddi_tile_launch(const float* s, const float* t, const int64_t* rel, int64_t n, int nc, const float* ff,
+                            const float* dd, int L, const float* gp, const float* gq, float* o1, float* o2,
+                            hipStream_t st) {
+    if constexpr (NC <= DDI_MAXC) {
+        if (nc != NC) return ddi_tile_launch<BWD, NC + 1>(s, t, rel, n, nc, ff, dd, L, gp, gq, o1, o2, st);
+        const int64_t bytes = ddi_tile_bytes(nc, L);
+        if (bytes > DDI_LDS_BYTES) return false;
+        // every tile starts at a multiple of 64 rows, so the arrays' own alignment is the rows'
+        uintptr_t al = reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(t);
+        if (BWD) al |= reinterpret_cast<uintptr_t>(o1) | reinterpret_cast<uintptr_t>(o2);
+        // resident blocks: 10 of 3 waves per CU (32 wave slots), 8 tiles or fewer each before more are added
+        const int64_t tiles = (n + DDI_PAIRS - 1) / DDI_PAIRS;
+        const unsigned grid = (unsigned)std::min<int64_t>(tiles, 256 * 10 * 4);
+        ddi_tile_kernel<NC, BWD><<<grid, DDI_THREADS, (size_t)bytes, st>>>(s, t, rel, n, ff, dd, L, al % 16 == 0, gp,
+                                                                           gq, o1, o2);
+        return true;
+    }
+    return false;
+}
 
 static unsigned ddi_grid(int64_t n) {
     const int64_t b = (n + 255) / 256;
@@ -371,10 +446,9 @@ int ngs_ddi_forward(const float* source_expanded, const float* target_expanded, 
     if (n <= 0) return NGS_OK;
     NGS_REQUIRE(source_expanded && target_expanded && rel_pos && f_f_i && df_df_i && p_mats && q_mats,
                 "ngs_ddi_forward: null argument");
-    if (ddi_use_lds(n_components, table_len) && ddi_tiled_bytes(n_components, table_len) <= DDI_LDS_BYTES)
-        ddi_forward_tiled_kernel<<<ddi_grid(n), DDI_TILE, (size_t)ddi_tiled_bytes(n_components, table_len), S(s)>>>(
-            source_expanded, target_expanded, rel_pos, n, n_components, f_f_i, df_df_i, table_len, p_mats, q_mats);
-    else if (ddi_use_lds(n_components, table_len))
+    if (ddi_tile_launch<false>(source_expanded, target_expanded, rel_pos, n, n_components, f_f_i, df_df_i, table_len,
+                               nullptr, nullptr, p_mats, q_mats, S(s))) {
+    } else if (ddi_use_lds(n_components, table_len))
         ddi_forward_lds_kernel<<<ddi_grid(n), 256, (size_t)n_components * n_components * table_len * 8, S(s)>>>(
             source_expanded, target_expanded, rel_pos, n, n_components, f_f_i, df_df_i, table_len, p_mats, q_mats);
     else
@@ -392,7 +466,9 @@ int ngs_ddi_backward(const float* source_expanded, const float* target_expanded,
     NGS_REQUIRE(source_expanded && target_expanded && rel_pos && f_f_i && df_df_i && grad_p && grad_q && grad_s &&
                     grad_t,
                 "ngs_ddi_backward: null argument");
-    if (ddi_use_lds(n_components, table_len))
+    if (ddi_tile_launch<true>(source_expanded, target_expanded, rel_pos, n, n_components, f_f_i, df_df_i, table_len,
+                              grad_p, grad_q, grad_s, grad_t, S(s))) {
+    } else if (ddi_use_lds(n_components, table_len))
         ddi_backward_lds_kernel<<<ddi_grid(n), 256, (size_t)n_components * n_components * table_len * 8, S(s)>>>(
             source_expanded, target_expanded, rel_pos, n, n_components, f_f_i, df_df_i, table_len, grad_p, grad_q,
             grad_s, grad_t);

@@ -292,6 +292,12 @@ class EvalDerivFunc(torch.autograd.Function):
         return None, g, None, None, None, None
 
 
+def _within(r, L):
+    """Whether every value of r lies in [0, L): one pass and one device-to-host read."""
+    lo, hi = torch.stack(torch.aminmax(r)).tolist()
+    return 0 <= lo and hi < L
+
+
 class DDIFunc(torch.autograd.Function):
     """Differentiable nabla B_k . nabla B_l factors (additive.py:55-68, ddi.cu), on the GPU."""
 
@@ -305,7 +311,7 @@ class DDIFunc(torch.autograd.Function):
         n, nc, L = s.shape[0], ff.shape[0], ff.shape[2]
         if s.shape != (n, 3 * nc) or t.shape != (n, 3 * nc) or r.shape != (n, 3) or dd.shape != ff.shape:
             raise NgsError("ddi_forward: inconsistent shapes")
-        if n and not (0 <= int(r.min()) and int(r.max()) < L):
+        if n and not _within(r, L):
             raise NgsError("ddi_forward: rel_pos outside the table")
         p = torch.empty((n, 3), dtype=torch.float32, device=s.device)
         q = torch.empty((n, 3), dtype=torch.float32, device=s.device)
