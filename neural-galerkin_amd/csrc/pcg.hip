@@ -77,6 +77,8 @@ struct PcgArgs {
     float* p;
     float* q;
     double* partials;  // 3 * nblocks: p.q | r.z | r.r (per block)
+    double* pq;        // partials of p.q the update step sums, and how many: partials and nblocks, or in
+    int npq;           // a wide solve the 2 nblocks behind the three arrays
     PcgState* st;
     int64_t M;
     int64_t chunk;     // rows per block
@@ -620,6 +622,106 @@ __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_e
     }
 }
 
+// ---- one slice over five waves
+// The same products and sums, bit for bit, with a slice's 5 plane batches loaded by 5 waves at once: two
+// memory round trips per slice (run words, then values and gathers together) instead of ten in a row. The
+// fused multiply-adds still run in plane order: wave k continues the sum that wave k - 1 leaves in LDS.
+// For systems that leave the chip waiting: up to 64k rows all slices are resident (2 per block of 10 waves,
+// 2 blocks per CU by LDS), 11.7 -> 6.0 us per product at 9.4k rows, 11.4 -> 9.6 at 64k; beyond that the
+// LDS hand-over costs more than the latency it hides (15.1 against 28.0 us at 132k rows). A whole Jacobi
+// iteration, with the block counts above and the shorter load chains below: 32.5 -> 14.4 us at 9.4k rows,
+// 30.2 -> 19.6 at 41k.
+constexpr int64_t WIDE_ROWS = 65536;
+constexpr int WIDE_GROUPS = 2;                        // slices in flight per block
+constexpr int WIDE_WAVES = 25 / PACK_BATCH;           // waves per slice
+constexpr int WIDE_THREADS = 64 * WIDE_WAVES * WIDE_GROUPS;
+
+struct WideLds {
+    float stage[WIDE_GROUPS * WIDE_WAVES][PACK_STAGE];
+    float carry[WIDE_GROUPS][64];
+    int tot[WIDE_GROUPS][WIDE_WAVES];
+};
+
+// Rows base .. base + 64 WIDE_GROUPS - 1 (base < M, uniform over the block; every thread calls). The row
+// sum is returned in the last wave of each slice.
+__device__ __forceinline__ float wide_row_dot(const NGS_GLOBAL int32_t* __restrict__ runs,
+                                              const NGS_GLOBAL float* __restrict__ pvals,
+                                              const NGS_GLOBAL int64_t* __restrict__ soff,
+                                              const NGS_GLOBAL float* __restrict__ x, int64_t P, int64_t M,
+                                              int64_t base, WideLds& lds) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane64();
+    const int grp = wave / WIDE_WAVES, wv = wave % WIDE_WAVES;
+    const int64_t row = base + 64 * grp + lane;
+    const bool ok = row < M;
+    const int64_t sl = base / 64 + grp;
+    int64_t pos = 64 * sl < M ? soff[sl] : 0;
+    int32_t w[PACK_BATCH];
+    int ex[PACK_BATCH];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b) w[b] = ok ? runs[(wv * PACK_BATCH + b) * P + row] : 0;
+    float xv[PACK_BATCH][5];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b) {
+        const int32_t start = w[b] & RUN_START_MASK;
+        const int n = (int)((uint32_t)w[b] >> RUN_COUNT_SHIFT);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) xv[b][j] = j < n ? x[start + j] : 0.f;
+    }
+    const int tot = batch_prefix5(w, ex);
+    if (lane == 0) lds.tot[grp][wv] = tot;
+    __syncthreads();
+    for (int u = 0; u < wv; ++u) pos += lds.tot[grp][u];
+    float* stage = lds.stage[wave];
+    {
+        float t[PACK_STAGE / 64];
+#pragma unroll
+        for (int u = 0; u < PACK_STAGE / 64; ++u) {
+            const int e = u * 64 + lane;
+            t[u] = (u * 64 < tot && e < tot) ? pvals[pos + e] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < PACK_STAGE / 64; ++u) {
+            const int e = u * 64 + lane;
+            if (u * 64 < tot && e < tot) stage[e] = t[u];
+        }
+    }
+    wave_lds_sync();
+    float v[PACK_BATCH][5];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b) {
+        const int n = (int)((uint32_t)w[b] >> RUN_COUNT_SHIFT);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) v[b][j] = j < n ? stage[ex[b] + j] : 0.f;
+    }
+    float sum = 0.f;
+    for (int k = 0; k < WIDE_WAVES; ++k) {
+        if (wv == k) {
+            if (k) sum = lds.carry[grp][lane];
+#pragma unroll
+            for (int b = 0; b < PACK_BATCH; ++b)
+#pragma unroll
+                for (int j = 0; j < 5; ++j) sum = __builtin_fmaf(v[b][j], xv[b][j], sum);
+            if (k < WIDE_WAVES - 1) lds.carry[grp][lane] = sum;
+        }
+        if (k < WIDE_WAVES - 1) __syncthreads();
+    }
+    return sum;
+}
+
+__global__ void __launch_bounds__(WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
+spmv_packed_wide_kernel(const int32_t* __restrict__ runs, const float* __restrict__ pvals,
+                        const int64_t* __restrict__ soff, const float* __restrict__ x, float* __restrict__ y,
+                        int64_t M) {
+    __shared__ WideLds lds;
+    const int64_t P = run_plane_stride(M);
+    const bool last = (threadIdx.x >> 6) % WIDE_WAVES == WIDE_WAVES - 1;
+    const int64_t base = (int64_t)blockIdx.x * 64 * WIDE_GROUPS;
+    if (base >= M) return;
+    const float sum = wide_row_dot(as_global(runs), as_global(pvals), as_global(soff), as_global(x), P, M, base, lds);
+    const int64_t row = base + 64 * (int64_t)((threadIdx.x >> 6) / WIDE_WAVES) + lane64();
+    if (last && row < M) y[row] = sum;
+}
+
 // r = b - A x in FP64 (FP32 entries, FP64 x and products), 8 lanes per row with 16-byte loads of
 // entries and columns. x == nullptr means x = 0 (r = b, no matrix pass).
 __global__ void __launch_bounds__(PCG_THREADS) residual_f64_kernel(const int32_t* __restrict__ rowptr,
@@ -794,13 +896,14 @@ __global__ void __launch_bounds__(PCG_THREADS) stencil_residual_kernel(ngs_stenc
 }
 
 static int pcg_blocks(int64_t M, int64_t* chunk) {
-    // ~256 rows per block (8 rows per 8-lane group): small levels get enough blocks that each
-    // group walks only a few rows, so their iterations are not bound by a long latency chain. At most
+    // 256 rows per block: small levels get enough blocks that each wave of the SpMV walks one slice, so
+    // their iterations are not bound by a long latency chain (rounding the count down to a multiple of 8
+    // instead left the first block a second slice: 24 us per product at 9k rows against 12). At most
     // 2560 = 2 x 256 CUs x 5: the grid-stride SpMV of large systems runs in two full rounds of resident
     // blocks (bpcg_packed_dot_kernel holds 5 blocks per CU)
     int64_t nb = (M + 255) / 256;
+    if (nb > NUM_XCD) nb = (nb + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
     if (nb > 2560) nb = 2560;
-    if (nb >= NUM_XCD) nb = (nb / NUM_XCD) * NUM_XCD;
     if (nb < 1) nb = 1;
     // whole 64-row groups per block: the vector loads and stores of each wave are aligned 256-byte
     // segments (the last blocks may get fewer rows, or none)
@@ -810,7 +913,7 @@ static int pcg_blocks(int64_t M, int64_t* chunk) {
 
 static size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 
-static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, int32_t** map = nullptr) {
+static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, bool wide = false) {
     int64_t chunk;
     int nb = pcg_blocks(M, &chunk);
     size_t off = 0;
@@ -818,6 +921,15 @@ static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, int
     off += al256(sizeof(PcgState));
     A->partials = reinterpret_cast<double*>(ws + off);
     off += al256(sizeof(double) * 3 * nb);
+    A->pq = A->partials;
+    A->npq = nb;
+    if (M <= WIDE_ROWS) {
+        if (wide) {
+            A->pq = reinterpret_cast<double*>(ws + off);
+            A->npq = 2 * nb;
+        }
+        off += al256(sizeof(double) * 2 * nb);
+    }
     A->r = reinterpret_cast<float*>(ws + off);
     off += al256(sizeof(float) * M);
     A->p = reinterpret_cast<float*>(ws + off);
@@ -825,8 +937,6 @@ static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, int
     A->q = reinterpret_cast<float*>(ws + off);
     off += al256(sizeof(float) * M);
     if (tab) *tab = ws + off;
-    off += 512;  // one batch table entry
-    if (map) *map = reinterpret_cast<int32_t*>(ws + off);
     A->nblocks = nb;
     A->chunk = chunk;
     A->M = M;
@@ -836,7 +946,8 @@ static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, int
 static int64_t pcg_ws_bytes(int64_t M) {
     int64_t chunk;
     int nb = pcg_blocks(M, &chunk);
-    return (int64_t)(al256(sizeof(PcgState)) + al256(sizeof(double) * 3 * nb) + 3 * al256(sizeof(float) * M) + 512 +
+    return (int64_t)(al256(sizeof(PcgState)) + al256(sizeof(double) * 3 * nb) +
+                     (M <= WIDE_ROWS ? al256(sizeof(double) * 2 * nb) : 0) + 3 * al256(sizeof(float) * M) + 512 +
                      al256(sizeof(int32_t) * nb));
 }
 
@@ -858,7 +969,9 @@ static HostState& host_state() {
 enum : int32_t { SYS_CSR = 0, SYS_STENCIL = 1, SYS_RUNS = 2, SYS_PACKED = 3 };
 
 // Flags of a launch sequence (which kernels the table's systems need).
-enum : int32_t { FLAG_STENCIL = 1, FLAG_RUNS = 2, FLAG_NO_CSR = 4, FLAG_PACKED = 8, FLAG_FILTER = 16 };
+enum : int32_t { FLAG_STENCIL = 1, FLAG_RUNS = 2, FLAG_NO_CSR = 4, FLAG_PACKED = 8, FLAG_FILTER = 16,
+// one packed system of at most WIDE_ROWS rows laid out for the wide product (internal)
+                 FLAG_WIDE = 32 };
 
 struct BatchSys {
     PcgArgs a;
@@ -870,7 +983,14 @@ struct BatchSys {
 };
 static_assert(sizeof(BatchSys) <= 512, "batch table entry must fit its workspace slot");
 
+// A null map: the table's first entry owns the whole grid (a solve of one system; the kernels of a small one
+// are chains of dependent loads, and this saves the first).
 __device__ __forceinline__ const BatchSys* batch_lookup(const BatchSys* tab, const int32_t* blk2sys, int* local) {
+    if (!blk2sys) {
+        const int nb = gridDim.x, lb = blockIdx.x;
+        *local = (nb % NUM_XCD) ? lb : (lb % NUM_XCD) * (nb / NUM_XCD) + lb / NUM_XCD;
+        return tab;
+    }
     const int sys = blk2sys[blockIdx.x];
     if (sys < 0) return nullptr;
     const BatchSys* B = tab + sys;
@@ -992,6 +1112,39 @@ __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_e
     store_partials2(pq, 0.0, A.partials, nullptr, lb);
 }
 
+// The same for a single system of at most WIDE_ROWS rows, a slice over five waves (wide_row_dot): 128 rows
+// and one partial per block, 2 nblk blocks.
+__global__ void __launch_bounds__(WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
+bpcg_packed_wide_dot_kernel(const BatchSys* tab, int ph) {
+    __shared__ WideLds lds;
+    __shared__ double part[WIDE_GROUPS];
+    const PcgArgs& A = tab->a;
+    const int64_t base = (int64_t)blockIdx.x * 64 * WIDE_GROUPS;
+    if (base >= A.M) {  // past the rows (the block count is a multiple of 8): an empty partial
+        if (threadIdx.x == 0) as_global(A.pq)[blockIdx.x] = 0.0;
+        return;
+    }
+    const int done = A.st->slot[ph].done;  // waited for below, with the product's first loads
+    const NGS_GLOBAL float* __restrict__ p = as_global(A.p);
+    const int grp = (threadIdx.x >> 6) / WIDE_WAVES;
+    const bool last = (threadIdx.x >> 6) % WIDE_WAVES == WIDE_WAVES - 1;
+    const int64_t row = base + 64 * grp + lane64();
+    const bool on = last && row < A.M;
+    const float prow = on ? p[row] : 0.f;
+    if (done) return;
+    const float sum = wide_row_dot(as_global(A.runs), as_global(A.rvals), as_global(A.soff), p, run_plane_stride(A.M),
+                                   A.M, base, lds);
+    if (on) as_global(A.q)[row] = sum;
+    const double pq = wave_sum(on ? (double)prow * sum : 0.0);
+    if (last && lane64() == 0) part[grp] = pq;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0;
+        for (int k = 0; k < WIDE_GROUPS; ++k) t += part[k];
+        as_global(A.pq)[blockIdx.x] = t;
+    }
+}
+
 // The same for the stencil systems of the table (row pass; the point pass ran before).
 __global__ void __launch_bounds__(PCG_THREADS) bpcg_stencil_dot_kernel(const BatchSys* tab, const int32_t* blk2sys,
                                                                        int ph) {
@@ -1042,11 +1195,12 @@ __global__ void __launch_bounds__(PCG_THREADS) bpcg_update_kernel(const BatchSys
     const BatchSys* B = batch_lookup(tab, blk2sys, &lb);
     if (!B) return;
     const PcgArgs& A = B->a;
-    if (A.st->slot[ph].done) return;
     const int nb = B->nblk;
     double* partials = A.partials;
+    const int done = A.st->slot[ph].done;  // read with the partials, not before them
     double pq, unused;
-    sum_partials2(partials, nullptr, nb, pq, unused);
+    sum_partials2(A.pq, nullptr, A.npq, pq, unused);
+    if (done) return;
     const float alpha = (float)(A.st->rz[ph] / pq);
     const int64_t r0 = (int64_t)lb * A.chunk;
     const int64_t r1 = min(A.M, r0 + A.chunk);
@@ -1145,15 +1299,18 @@ __global__ void __launch_bounds__(PCG_THREADS) bpcg_direction_kernel(const Batch
     if (!B) return;
     const PcgArgs& A = B->a;
     PcgState* st = A.st;
-    if (st->slot[ph].done) return;
     const int nb = B->nblk;
+    const PcgSlot sl = st->slot[ph];  // the state is read with the partials, not before them
+    const double stop = st->tol2 * st->bb, rz_old = st->rz[ph];
+    const int max_iter = st->max_iter;
     double rz_new, rr;
     sum_partials2(A.partials + nb, A.partials + 2 * nb, nb, rz_new, rr);
-    const int it = st->slot[ph].iter + 1;
-    const bool conv = rr <= st->tol2 * st->bb;
-    const bool cap = !conv && it >= st->max_iter;
+    if (sl.done) return;
+    const int it = sl.iter + 1;
+    const bool conv = rr <= stop;
+    const bool cap = !conv && it >= max_iter;
     if (!conv && !cap) {
-        const float beta = (float)(rz_new / st->rz[ph]);
+        const float beta = (float)(rz_new / rz_old);
         const int64_t r0 = (int64_t)lb * A.chunk;
         const int64_t r1 = min(A.M, r0 + A.chunk);
         NGS_GLOBAL float* __restrict__ p = as_global(A.p);
@@ -1209,11 +1366,6 @@ __global__ void __launch_bounds__(PCG_THREADS) bpcg_direction_kernel(const Batch
 
 __global__ void write_entry_kernel(BatchSys* dst, BatchSys src) { *dst = src; }
 
-__global__ void fill_map_kernel(int32_t* map, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) map[i] = 0;
-}
-
 // SpMV variant: lanes per row (8, 16, 32), non-temporal matrix loads and interleaved row tiles;
 // set by ngs_pcg_config.
 static int g_spmv_lanes = 8;
@@ -1250,7 +1402,8 @@ static void launch_batch_iteration(const BatchSys* tab, const int32_t* blk2sys, 
         });
     }
     if (flags & FLAG_RUNS) bpcg_runs_dot_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
-    if (flags & FLAG_PACKED) bpcg_packed_dot_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
+    if (flags & FLAG_WIDE) bpcg_packed_wide_dot_kernel<<<2 * total_blocks, WIDE_THREADS, 0, st>>>(tab, ph);
+    else if (flags & FLAG_PACKED) bpcg_packed_dot_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
     if (flags & FLAG_STENCIL) bpcg_stencil_dot_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
     bpcg_update_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
     if (flags & FLAG_FILTER) bpcg_filter_kernel<<<grid, block, 0, st>>>(tab, blk2sys, ph);
@@ -1264,8 +1417,8 @@ using namespace ngs;
 extern "C" {
 
 int64_t ngs_pcg_workspace_bytes(int64_t M) { return pcg_ws_bytes(M); }
-int ngs_pcg_batch_iterate(const void* table, const int32_t* blk2sys, int32_t total_blocks, int32_t iters,
-                          int32_t use_graph, int32_t flags, ngs_stream_t s);
+static int batch_iterate(const BatchSys* tab, const int32_t* blk2sys, int32_t total_blocks, int32_t iters,
+                         int32_t use_graph, int32_t flags, hipStream_t st);
 
 // Environment-free knobs for measurement: graph use and lanes per row (0 = automatic).
 static int g_pcg_use_graph = 1;
@@ -1281,7 +1434,7 @@ int ngs_pcg_config(int32_t use_graph, int32_t lanes_per_row, int32_t nontemporal
     return NGS_OK;
 }
 
-// One system through the table-driven kernels: the single-entry table and its block map live in
+// One system through the table-driven kernels: the single-entry table lives in
 // the workspace, so the captured chunk graph depends only on (workspace, blocks, chunk) and is
 // replayed by every later solve that reuses the workspace.
 static int pcg_solve_entry(BatchSys E, int64_t M, double tol, int32_t max_iter, int32_t chunk, void* workspace,
@@ -1300,9 +1453,9 @@ static int pcg_solve_entry(BatchSys E, int64_t M, double tol, int32_t max_iter, 
     NGS_CHECK_HIP(hipEventRecord(ev, st));
     NGS_CHECK_HIP(hipStreamWaitEvent(work, ev, 0));
     void* tab = nullptr;
-    int32_t* map = nullptr;
     PcgArgs A = E.a;
-    pcg_layout(M, &A, reinterpret_cast<char*>(workspace), &tab, &map);
+    const bool wide = E.kind == SYS_PACKED && M <= WIDE_ROWS;
+    pcg_layout(M, &A, reinterpret_cast<char*>(workspace), &tab, wide);
     pcg_init_kernel<<<A.nblocks, PCG_THREADS, 0, work>>>(A);
     if (A.fwords) pcg_init_filter_kernel<<<A.nblocks, PCG_THREADS, 0, work>>>(A);
     pcg_init_finish_kernel<<<1, PCG_THREADS, 0, work>>>(A, tol, max_iter);
@@ -1310,18 +1463,17 @@ static int pcg_solve_entry(BatchSys E, int64_t M, double tol, int32_t max_iter, 
     E.blk0 = 0;
     E.nblk = A.nblocks;
     write_entry_kernel<<<1, 1, 0, work>>>(reinterpret_cast<BatchSys*>(tab), E);
-    fill_map_kernel<<<grid1d(A.nblocks, 256), 256, 0, work>>>(map, A.nblocks);
     NGS_CHECK_LAUNCH();
     const int flags = E.kind == SYS_STENCIL ? (FLAG_STENCIL | FLAG_NO_CSR)
                       : E.kind == SYS_RUNS ? (FLAG_RUNS | FLAG_NO_CSR)
-                      : E.kind == SYS_PACKED ? (FLAG_PACKED | FLAG_NO_CSR | (E.a.fwords ? FLAG_FILTER : 0))
+                      : E.kind == SYS_PACKED ? (FLAG_PACKED | FLAG_NO_CSR | (E.a.fwords ? FLAG_FILTER : 0) | (wide ? FLAG_WIDE : 0))
                                              : 0;
     int status = NGS_OK;
     int32_t it = 0, done = 0;
     double sc[2];
     while (true) {
-        int r = ngs_pcg_batch_iterate(tab, map, A.nblocks, chunk, g_pcg_use_graph, flags,
-                                      reinterpret_cast<ngs_stream_t>(work));
+        int r = batch_iterate(reinterpret_cast<const BatchSys*>(tab), nullptr, A.nblocks, chunk, g_pcg_use_graph, flags,
+                              work);
         if (r != NGS_OK) return r;
         // one read per chunk: rr, bb and slot 0 (iteration count, done flag)
         NGS_CHECK_HIP(hipMemcpyAsync(hs.pinned, &A.st->rr, kStatusBytes, hipMemcpyDeviceToHost, work));
@@ -1466,7 +1618,7 @@ int ngs_pcg_solve_runs_noalloc(const int32_t* runs, const float* rvals, const fl
     hipStream_t st = S(s);
     // Everything runs on the caller's stream, launched directly (no private stream, event or graph).
     // The init kernels write every workspace word the iterations read before they read it: x, r, p,
-    // the r.z / b.b partials, the state of both slots, the table entry and the block map.
+    // the r.z / b.b partials, the state of both slots and the table entry.
     BatchSys E{};
     E.kind = SYS_RUNS;
     E.a.runs = runs;
@@ -1475,22 +1627,22 @@ int ngs_pcg_solve_runs_noalloc(const int32_t* runs, const float* rvals, const fl
     E.a.b = b;
     E.a.x = x;
     void* tab = nullptr;
-    int32_t* map = nullptr;
     PcgArgs A = E.a;
-    pcg_layout(M, &A, reinterpret_cast<char*>(ws), &tab, &map);
+    pcg_layout(M, &A, reinterpret_cast<char*>(ws), &tab);
     pcg_init_kernel<<<A.nblocks, PCG_THREADS, 0, st>>>(A);
     pcg_init_finish_kernel<<<1, PCG_THREADS, 0, st>>>(A, tol, max_iter);
     E.a = A;
     E.blk0 = 0;
     E.nblk = A.nblocks;
     write_entry_kernel<<<1, 1, 0, st>>>(reinterpret_cast<BatchSys*>(tab), E);
-    fill_map_kernel<<<grid1d(A.nblocks, 256), 256, 0, st>>>(map, A.nblocks);
     NGS_CHECK_LAUNCH();
     PcgSlot slot{};
     double sc[2];
     alignas(8) char status_bytes[kStatusBytes];
     while (true) {
-        if (int r = ngs_pcg_batch_iterate(tab, map, A.nblocks, chunk, 0, FLAG_RUNS | FLAG_NO_CSR, s)) return r;
+        if (int r = batch_iterate(reinterpret_cast<const BatchSys*>(tab), nullptr, A.nblocks, chunk, 0,
+                                  FLAG_RUNS | FLAG_NO_CSR, st))
+            return r;
         // one read per chunk: rr, bb and slot 0 (iteration count, done flag)
         NGS_CHECK_HIP(hipMemcpyAsync(status_bytes, &A.st->rr, kStatusBytes, hipMemcpyDeviceToHost, st));
         NGS_CHECK_HIP(hipStreamSynchronize(st));
@@ -1589,7 +1741,10 @@ int ngs_spmv_packed(const int32_t* runs, const float* pvals, const int64_t* soff
     NGS_REQUIRE(M <= RUN_START_MASK + 1, "ngs_spmv_packed: too many rows for run words");
     const int64_t groups = ((M + 63) / 64 + 3) / 4;
     const int nb = (int)std::min<int64_t>(groups, 8192);
-    spmv_packed_kernel<<<nb, PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
+    if (M <= WIDE_ROWS)
+        spmv_packed_wide_kernel<<<grid1d(M, 64 * WIDE_GROUPS), WIDE_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
+    else
+        spmv_packed_kernel<<<nb, PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }
@@ -1866,8 +2021,12 @@ int ngs_pcg_batch_iterate(const void* table, const int32_t* blk2sys, int32_t tot
                           int32_t use_graph, int32_t flags, ngs_stream_t s) {
     NGS_REQUIRE(table && blk2sys && total_blocks > 0 && iters > 0 && iters % 2 == 0,
                 "ngs_pcg_batch_iterate: bad arguments (iters must be even and positive)");
-    const BatchSys* tab = reinterpret_cast<const BatchSys*>(table);
-    hipStream_t st = S(s);
+    return batch_iterate(reinterpret_cast<const BatchSys*>(table), blk2sys, total_blocks, iters, use_graph,
+                         flags & ~FLAG_WIDE, S(s));
+}
+
+static int batch_iterate(const BatchSys* tab, const int32_t* blk2sys, int32_t total_blocks, int32_t iters,
+                         int32_t use_graph, int32_t flags, hipStream_t st) {
     if (!use_graph) {
         for (int i = 0; i < iters; ++i) launch_batch_iteration(tab, blk2sys, total_blocks, flags, i & 1, st);
         NGS_CHECK_LAUNCH();
@@ -1881,7 +2040,7 @@ int ngs_pcg_batch_iterate(const void* table, const int32_t* blk2sys, int32_t tot
     static thread_local std::vector<Key> cache;
     hipGraphExec_t exec = nullptr;
     for (auto& k : cache)
-        if (k.t == table && k.m == blk2sys && k.nb == total_blocks && k.it == iters && k.fl == flags && k.var == var &&
+        if (k.t == tab && k.m == blk2sys && k.nb == total_blocks && k.it == iters && k.fl == flags && k.var == var &&
             k.s == st)
             exec = k.e;
     if (!exec) {
@@ -1895,7 +2054,7 @@ int ngs_pcg_batch_iterate(const void* table, const int32_t* blk2sys, int32_t tot
             (void)hipGraphExecDestroy(cache.front().e);
             cache.erase(cache.begin());
         }
-        cache.push_back({table, blk2sys, total_blocks, iters, flags, var, st, exec});
+        cache.push_back({tab, blk2sys, total_blocks, iters, flags, var, st, exec});
     }
     NGS_CHECK_HIP(hipGraphLaunch(exec, st));
     return NGS_OK;
