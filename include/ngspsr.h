@@ -179,6 +179,14 @@ int ngs_splat_gather(ngs_grid g, const int32_t *node_coords, int64_t count, cons
  * the derivative with respect to q (finest-voxel units), as evaluate_derivative returns it. */
 int ngs_eval_field(ngs_grid g, const float *field, const float *xyz, int64_t n, float inv_voxel_size,
                    float scale, int32_t accumulate, float *out, float *grad_out, ngs_stream_t s);
+/* ngs_eval_field without gradient, queries processed in the order of the permutation `order` (n int32): the
+ * same values (out stays in query order), faster when `order` brings neighbouring queries together. */
+int ngs_eval_field_ordered(ngs_grid g, const float *field, const float *xyz, const int32_t *order, int64_t n,
+                           float inv_voxel_size, float scale, int32_t accumulate, float *out, ngs_stream_t s);
+/* Byte offset, in the workspace of the ngs_splat_gather call that just ran with the same sizes, of the
+ * permutation (n int32) that sorts its points by the lower node of their stencil; -1 where the call has
+ * no workspace. */
+int64_t ngs_splat_gather_order_offset(int64_t n, int64_t count);
 /* ngs_eval_field with accumulate = 1 and no gradient, for the points binned at the field's level by
  * ngs_bin_points (point_cell, basis in bin order, perm): slot k adds to out[perm[k]]. Bit-identical to
  * ngs_eval_field on the same points; the bitmap and coefficient reads follow the bins. */

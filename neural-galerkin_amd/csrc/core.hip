@@ -1,6 +1,8 @@
 // Keys, cuckoo table, ordered bitmap sets, scans, density/levels, splat and field evaluation.
 #include "common.h"
 
+#include <type_traits>
+
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -591,28 +593,47 @@ __global__ void splat_bins_kernel(const uint32_t* __restrict__ ks, const int32_t
     }
 }
 
-__global__ void splat_gather_kernel(ngs_grid g, const int32_t* __restrict__ nodes, int64_t count, float inv_vs,
-                                    int ncomp, const int32_t* __restrict__ bstart, const int32_t* __restrict__ bend,
-                                    const float* __restrict__ bxyz, const float* __restrict__ brow, double post,
-                                    double* __restrict__ acc) {
+// G lanes per node (1, or 4 S): lane (column, sub) takes the two bins of one (ox, oy) column and every S-th
+// point of them; the FP64 sums of the lanes are then added pairwise. One lane per node waits through its 8
+// bins in a row: right where the nodes fill the chip by themselves and most bins are empty or nearly so,
+// but on grids coarse against the points (the density grid, the coarse levels) there are too few nodes to
+// hide it. Measured, us for 1 / 4 / 16 / 64 lanes:
+//   16.1M nodes, 2.9M points: 934 1192 3472 -     821k nodes, 270k points: 74 77 149 498
+//   220k nodes, 2M points: 348 206 136 142        51k nodes, 300k points: 214 77 34 31
+//   10k nodes, 9k points on one side: 391 137 45 14        6.2k nodes, 100k points: 535 149 40 14
+template <int G>
+__global__ void __launch_bounds__(256) splat_gather_kernel(ngs_grid g, const int32_t* __restrict__ nodes, int64_t count,
+                                                           float inv_vs, int ncomp, const int32_t* __restrict__ bstart,
+                                                           const int32_t* __restrict__ bend,
+                                                           const float* __restrict__ bxyz,
+                                                           const float* __restrict__ brow, double post,
+                                                           double* __restrict__ acc) {
 #pragma clang fp contract(off)
-    const int64_t node = xcd_contiguous_block() * blockDim.x + threadIdx.x;
-    if (node >= count) return;
+    constexpr int C = G < 4 ? G : 4, S = G / C;  // columns side by side, lanes per column
+    const int64_t node = xcd_contiguous_block() * (256 / G) + threadIdx.x / G;
+    if (node >= count) return;  // uniform over the node's lanes
+    const int sub = threadIdx.x % S;
     const int s = 1 << g.log2_stride;
     const float inv_s = 1.0f / (float)s;
     const int N[3] = {nodes[3 * node], nodes[3 * node + 1], nodes[3 * node + 2]};
     const int lx = (N[0] >> g.log2_stride) - g.origin[0], ly = (N[1] >> g.log2_stride) - g.origin[1],
               lz = (N[2] >> g.log2_stride) - g.origin[2];
     double sum[3] = {0.0, 0.0, 0.0};
-    // the 8 bins with lower node N - (ox, oy, oz) s: one column query per (ox, oy) covers oz = 1, 0
-    for (int oxy = 0; oxy < 4; ++oxy) {
-        int32_t r0;
+    // the bins with lower node N - (ox, oy, oz) s, oz = 1, 0: one column query, both bins' bounds together
+    for (int oxy = (threadIdx.x % G) / S; oxy < 4; oxy += C) {
+        int32_t r0 = 0;
         const uint32_t m = grid_column(g, lx - (oxy >> 1), ly - (oxy & 1), lz - 1, 2, &r0);
+        int32_t js[2] = {0, 0}, je[2] = {0, 0};
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if ((m >> k) & 1u) {
+                const int32_t r = r0 + (k ? (int)(m & 1u) : 0);
+                js[k] = bstart[r];
+                je[k] = bend[r];
+            }
+#pragma unroll
         for (int k = 0; k < 2; ++k) {
-            if (!((m >> k) & 1u)) continue;
-            const int32_t r = r0 + __popc(m & ((1u << k) - 1u));
-            const int32_t e = bend[r];
-            for (int32_t j = bstart[r]; j < e; ++j) {
+            for (int32_t j = js[k] + sub; j < je[k]; j += S) {
                 int dc[3], sg[3];
                 float loc[3];
 #pragma unroll
@@ -639,47 +660,104 @@ __global__ void splat_gather_kernel(ngs_grid g, const int32_t* __restrict__ node
             }
         }
     }
-    if (ncomp) {
-        for (int c = 0; c < ncomp; ++c) acc[node * ncomp + c] += sum[c];
-    } else {
-        acc[node] += sum[0];
+    const int nc = ncomp ? ncomp : 1;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (c >= nc) break;
+#pragma unroll
+        for (int d = G / 2; d > 0; d >>= 1) sum[c] += __shfl_xor(sum[c], d, G);
+        if (threadIdx.x % G == 0) acc[node * nc + c] += sum[c];
     }
 }
 
-__global__ void eval_field_kernel(ngs_grid g, const float* __restrict__ field, const float* __restrict__ xyz, int64_t n,
-                                  float inv_vs, float scale, int accumulate, float* __restrict__ out,
-                                  float* __restrict__ grad) {
+// Members of g (its last rank).
+__device__ __forceinline__ int32_t grid_count(const ngs_grid& g) {
+    return as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
+}
+
+// Coefficients of the three columns (lx, ly - 1 .. ly + 1, lz - 1 .. lz + 1) around a cell, 0 where absent:
+// the columns' bitmap words together, then their ranks, then one 12-byte load per column (its present
+// voxels have consecutive ranks). Three waits for three columns instead of two for each, and a third of the
+// coefficient loads: scattered queries are bound by the cache lines their loads touch. `count`: grid_count.
+__device__ __forceinline__ void field_columns(const ngs_grid& g, const NGS_GLOBAL float* __restrict__ field,
+                                              int32_t count, int lx, int ly, int lz, float (&f)[3][3]) {
+    uint32_t m[3];
+    int32_t id[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        id[k] = 0;
+        m[k] = grid_column(g, lx, ly + k - 1, lz - 1, 3, &id[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        f[k][0] = f[k][1] = f[k][2] = 0.f;
+        if (!m[k]) continue;
+        // the load starts at the column's first coefficient, or 3 before the end
+        const int32_t at = max(0, min(id[k], count - 3));
+        float t0, t1, t2;
+        if (count >= 3) {
+            t0 = field[at];
+            t1 = field[at + 1];
+            t2 = field[at + 2];
+        } else {
+            t0 = field[0];
+            t1 = field[min(1, count - 1)];
+            t2 = t1;
+        }
+        int o = id[k] - at;
+#pragma unroll
+        for (int kz = 0; kz < 3; ++kz)
+            if ((m[k] >> kz) & 1u) {
+                f[k][kz] = o == 0 ? t0 : o == 1 ? t1 : t2;
+                ++o;
+            }
+    }
+}
+
+// order: a permutation of the queries (null: none); slot i evaluates query order[i]. Queries sorted by cell
+// read the bitmap and the coefficients of their neighbourhood together.
+template <bool GRAD>
+__global__ void __launch_bounds__(256) eval_field_kernel(ngs_grid g, const float* __restrict__ field,
+                                                         const float* __restrict__ xyz,
+                                                         const int32_t* __restrict__ order, int64_t n, float inv_vs,
+                                                         float scale, int accumulate, float* __restrict__ out,
+                                                         float* __restrict__ grad) {
 #pragma clang fp contract(off)
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (order) i = order[i];
     const int s = 1 << g.log2_stride;
     const float inv_s = 1.0f / (float)s;
+    const int32_t count = grid_count(g);
     int cell[3];
     float b[3][3], db[3][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) axis_basis_grad(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a], db[a]);
+    for (int a = 0; a < 3; ++a) {
+        if (GRAD) axis_basis_grad(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a], db[a]);
+        else axis_basis(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a]);
+    }
     float v = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
     const int l2 = g.log2_stride;
     const int lx = (cell[0] >> l2) - g.origin[0], ly = (cell[1] >> l2) - g.origin[1], lz = (cell[2] >> l2) - g.origin[2];
-    // the 27 voxels around the cell in (kx, ky, kz) order, one bitmap column per (kx, ky)
-    for (int kx = 0; kx < 3; ++kx)
-        for (int ky = 0; ky < 3; ++ky) {
-            int32_t id;
-            const uint32_t m = grid_column(g, lx + kx - 1, ly + ky - 1, lz - 1, 3, &id);
-            if (!m) continue;
+    // the 27 voxels around the cell in (kx, ky, kz) order (absent ones add 0)
+#pragma unroll
+    for (int kx = 0; kx < 3; ++kx) {
+        float f[3][3];
+        field_columns(g, as_global(field), count, lx + kx - 1, ly, lz, f);
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
             for (int kz = 0; kz < 3; ++kz) {
-                if (!((m >> kz) & 1u)) continue;
-                float f = field[id++];
-                v += (b[0][kx] * b[1][ky] * b[2][kz]) * f;
-                if (grad) {
-                    gx += (db[0][kx] * b[1][ky] * b[2][kz]) * f;
-                    gy += (b[0][kx] * db[1][ky] * b[2][kz]) * f;
-                    gz += (b[0][kx] * b[1][ky] * db[2][kz]) * f;
+                v += (b[0][kx] * b[1][ky] * b[2][kz]) * f[ky][kz];
+                if (GRAD) {
+                    gx += (db[0][kx] * b[1][ky] * b[2][kz]) * f[ky][kz];
+                    gy += (b[0][kx] * db[1][ky] * b[2][kz]) * f[ky][kz];
+                    gz += (b[0][kx] * b[1][ky] * db[2][kz]) * f[ky][kz];
                 }
             }
-        }
+    }
     out[i] = (accumulate ? out[i] : 0.f) + v * scale;
-    if (grad) {
+    if (GRAD) {
         float* gp = grad + 3 * i;
         gp[0] = (accumulate ? gp[0] : 0.f) + gx * scale;
         gp[1] = (accumulate ? gp[1] : 0.f) + gy * scale;
@@ -691,29 +769,30 @@ __global__ void eval_field_kernel(ngs_grid g, const float* __restrict__ field, c
 // and basis values come from the bins (point_basis_kernel's, the values axis_basis gives here too), the
 // 27 terms are summed in the same order, and slot k adds to out[perm[k]] (original point order), so
 // the result is bit-identical while the bitmap and coefficient reads follow the bins.
-__global__ void eval_field_binned_kernel(ngs_grid g, const float* __restrict__ field, const int32_t* __restrict__ cell,
-                                         const float* __restrict__ b, const int32_t* __restrict__ perm, int64_t n,
-                                         float scale, float* __restrict__ out) {
+__global__ void __launch_bounds__(256) eval_field_binned_kernel(ngs_grid g, const float* __restrict__ field,
+                                                                const int32_t* __restrict__ cell,
+                                                                const float* __restrict__ b,
+                                                                const int32_t* __restrict__ perm, int64_t n,
+                                                                float scale, float* __restrict__ out) {
 #pragma clang fp contract(off)
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
+    const int64_t p = perm[k];
     const float* bk = b + 9 * k;
     const int l2 = g.log2_stride;
+    const int32_t count = grid_count(g);
     const int lx = (cell[3 * k] >> l2) - g.origin[0], ly = (cell[3 * k + 1] >> l2) - g.origin[1],
               lz = (cell[3 * k + 2] >> l2) - g.origin[2];
     float v = 0.f;
-    for (int kx = 0; kx < 3; ++kx)
-        for (int ky = 0; ky < 3; ++ky) {
-            int32_t id;
-            const uint32_t m = grid_column(g, lx + kx - 1, ly + ky - 1, lz - 1, 3, &id);
-            if (!m) continue;
-            for (int kz = 0; kz < 3; ++kz) {
-                if (!((m >> kz) & 1u)) continue;
-                const float f = field[id++];
-                v += (bk[kx] * bk[3 + ky] * bk[6 + kz]) * f;
-            }
-        }
-    const int64_t p = perm[k];
+#pragma unroll
+    for (int kx = 0; kx < 3; ++kx) {
+        float f[3][3];
+        field_columns(g, as_global(field), count, lx + kx - 1, ly, lz, f);
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+            for (int kz = 0; kz < 3; ++kz) v += (bk[kx] * bk[3 + ky] * bk[6 + kz]) * f[ky][kz];
+    }
     out[p] = out[p] + v * scale;
 }
 
@@ -1176,8 +1255,16 @@ int ngs_splat_gather(ngs_grid g, const int32_t* node_coords, int64_t count, cons
     splat_bins_kernel<<<grid1d(n, 256), 256, 0, st>>>(ks, order, n, (uint32_t)count, xyz, data, ncomp, scale, bstart,
                                                       bend, bxyz, brow);
     NGS_CHECK_LAUNCH();
-    splat_gather_kernel<<<grid1d(count, 256), 256, 0, st>>>(g, node_coords, count, inv_voxel_size, data ? ncomp : 0,
-                                                            bstart, bend, bxyz, brow, post, acc);
+    // lanes per node: enough threads for the chip (500k resident), see the kernel's figures
+    auto gather = [&](auto lanes) {
+        constexpr int G = decltype(lanes)::value;
+        splat_gather_kernel<G><<<grid1d(count, 256 / G), 256, 0, st>>>(
+            g, node_coords, count, inv_voxel_size, data ? ncomp : 0, bstart, bend, bxyz, brow, post, acc);
+    };
+    if (count > 1500000) gather(std::integral_constant<int, 1>());
+    else if (count > 400000) gather(std::integral_constant<int, 4>());
+    else if (count > 12000) gather(std::integral_constant<int, 16>());
+    else gather(std::integral_constant<int, 64>());
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }
@@ -1185,9 +1272,31 @@ int ngs_splat_gather(ngs_grid g, const int32_t* node_coords, int64_t count, cons
 int ngs_eval_field(ngs_grid g, const float* field, const float* xyz, int64_t n, float inv_voxel_size, float scale,
                    int32_t accumulate, float* out, float* grad_out, ngs_stream_t s) {
     if (n <= 0) return NGS_OK;
-    eval_field_kernel<<<grid1d(n, 256), 256, 0, S(s)>>>(g, field, xyz, n, inv_voxel_size, scale, accumulate, out, grad_out);
+    if (grad_out)
+        eval_field_kernel<true><<<grid1d(n, 256), 256, 0, S(s)>>>(g, field, xyz, nullptr, n, inv_voxel_size, scale,
+                                                                  accumulate, out, grad_out);
+    else
+        eval_field_kernel<false><<<grid1d(n, 256), 256, 0, S(s)>>>(g, field, xyz, nullptr, n, inv_voxel_size, scale,
+                                                                   accumulate, out, nullptr);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
+}
+
+int ngs_eval_field_ordered(ngs_grid g, const float* field, const float* xyz, const int32_t* order, int64_t n,
+                           float inv_voxel_size, float scale, int32_t accumulate, float* out, ngs_stream_t s) {
+    if (n <= 0) return NGS_OK;
+    NGS_REQUIRE(xyz && order && out, "ngs_eval_field_ordered: null argument");
+    eval_field_kernel<false><<<grid1d(n, 256), 256, 0, S(s)>>>(g, field, xyz, order, n, inv_voxel_size, scale,
+                                                               accumulate, out, nullptr);
+    NGS_CHECK_LAUNCH();
+    return NGS_OK;
+}
+
+int64_t ngs_splat_gather_order_offset(int64_t n, int64_t count) {
+    if (n <= 0 || count <= 0 || count >= ((int64_t)1 << 31) || n >= ((int64_t)1 << 31)) return -1;
+    size_t tmp, off[8], total;
+    if (splat_gather_layout(n, count, &tmp, off, &total) != NGS_OK) return -1;
+    return (int64_t)off[3];
 }
 
 int ngs_eval_field_binned(ngs_grid g, const float* field, const int32_t* point_cell, const float* basis,

@@ -303,11 +303,16 @@ class HashTree:
         q4min, q4max = self._bounds(inv4)
         g4 = self._voxelise(1, inv4, q4min, q4max)
         w = torch.zeros(g4.count, dtype=torch.float64, device=self.device)
-        self._splat(g4, self.xyz, inv4, None, 0, None, None, 0, w)
+        order = self._splat(g4, self.xyz, inv4, None, 0, None, None, 0, w)
         wf = w.float()
-        rho = torch.empty(self.xyz.shape[0], dtype=torch.float32, device=self.device)
-        call("ngs_eval_field", g4.struct(), ptr(wf), ptr(self.xyz), self.xyz.shape[0], inv4, 1.0 / (enc * enc), 0,
-             ptr(rho), None, stream())
+        n = self.xyz.shape[0]
+        rho = torch.empty(n, dtype=torch.float32, device=self.device)
+        if order is not None:  # the points in the order of the splat's sort
+            call("ngs_eval_field_ordered", g4.struct(), ptr(wf), ptr(self.xyz), ptr(order), n, inv4, 1.0 / (enc * enc),
+                 0, ptr(rho), stream())
+        else:
+            call("ngs_eval_field", g4.struct(), ptr(wf), ptr(self.xyz), n, inv4, 1.0 / (enc * enc), 0, ptr(rho), None,
+                 stream())
         return rho
 
     def _set_encoder_levels(self, grids):
@@ -456,16 +461,20 @@ class HashTree:
     # ------------------------------------------------------------------ data on the tree
     def _splat(self, g, xyz, inv_vs, data, nc, scale, levels, level, out):
         """acc += the trilinear splat of the points on g: the binned gather (no FP64 atomics), or the
-        atomic scatter where g's members are not emitted or the sizes exceed the gather's."""
+        atomic scatter where g's members are not emitted or the sizes exceed the gather's. Returns the
+        permutation the gather sorted the points by (a view of the thread's scratch, valid until its
+        next use), or None."""
         n = xyz.shape[0]
         wsb = lib().ngs_splat_gather_workspace_bytes(n, g.count) if g.coords is not None else -1
         if wsb < 0:
             call("ngs_splat", g.struct(), ptr(xyz), n, inv_vs, ptr(data), nc, ptr(scale), ptr(levels), level, 1.0,
                  ptr(out), stream())
-            return
+            return None
         ws = Scratch.get(wsb, self.device)
         call("ngs_splat_gather", g.struct(), ptr(g.coords), g.count, ptr(xyz), n, inv_vs, ptr(data), nc, ptr(scale),
              ptr(levels), level, 1.0, ptr(out), ptr(ws), wsb, stream())
+        off = int(lib().ngs_splat_gather_order_offset(n, g.count))
+        return ws[off:off + 4 * n].view(torch.int32) if off >= 0 else None
 
     def splat_data(self, xyz, branch, data_depth, data=None, check_corr=True, scale=None, levels=None, level=0):
         """_hash_backend.py:332-356 (float64 accumulation, returned as float32), rows in the level's
