@@ -457,26 +457,6 @@ __global__ void __launch_bounds__(PCG_THREADS) runs_slice_counts_kernel(const in
     if (lane64() == 0) counts[sl] = tot;
 }
 
-// Slot form -> packed form. One wave per slice.
-__global__ void __launch_bounds__(PCG_THREADS) runs_pack_kernel(const int32_t* __restrict__ runs,
-                                                                const float* __restrict__ rvals, int64_t M,
-                                                                const int64_t* __restrict__ soff,
-                                                                float* __restrict__ pvals) {
-    const int64_t nsl = (M + 63) / 64;
-    const int64_t sl = ((int64_t)blockIdx.x * PCG_THREADS + threadIdx.x) >> 6;
-    if (sl >= nsl) return;
-    const int64_t row = sl * 64 + lane64();
-    const int64_t P = run_plane_stride(M);
-    int64_t pos = soff[sl];
-    for (int p = 0; p < 25; ++p) {
-        const int n = row < M ? (int)((uint32_t)runs[p * P + row] >> RUN_COUNT_SHIFT) : 0;
-        int ex, t;
-        wave_prefix3(n, ex, t);
-        for (int j = 0; j < n; ++j) pvals[pos + ex + j] = rvals[(5 * p + j) * P + row];
-        pos += t;
-    }
-}
-
 // Packed form -> slot form (the inverse of runs_pack_kernel; slots past a run hold 0).
 __global__ void __launch_bounds__(PCG_THREADS) runs_unpack_kernel(const int32_t* __restrict__ runs,
                                                                   const float* __restrict__ pvals, int64_t M,
@@ -531,6 +511,41 @@ __device__ __forceinline__ int batch_prefix5(const int32_t (&w)[5], int (&ex)[5]
     ex[3] = T0 + T1 + T2 + (e1 & 511);
     ex[4] = T0 + T1 + T2 + T3 + ((e1 >> 9) & 511);
     return T0 + T1 + T2 + T3 + T4;
+}
+
+// Slot form -> packed form. One block of 5 waves per slice, a wave per batch of 5 planes (batch_prefix5), so the
+// 25 planes are not one chain of loads, ballots and stores: 45 us for any level under 50k rows with one wave
+// per slice.
+constexpr int PACK_WAVES = 25 / PACK_BATCH;
+__global__ void __launch_bounds__(64 * PACK_WAVES) runs_pack_kernel(const int32_t* __restrict__ runs,
+                                                                    const float* __restrict__ rvals, int64_t M,
+                                                                    const int64_t* __restrict__ soff,
+                                                                    float* __restrict__ pvals) {
+    __shared__ int tots[PACK_WAVES];
+    const int64_t sl = blockIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = sl * 64 + lane64();
+    const int64_t P = run_plane_stride(M);
+    int64_t pos = soff[sl];
+    int32_t w[PACK_BATCH];
+    int ex[PACK_BATCH];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b) w[b] = row < M ? runs[(wv * PACK_BATCH + b) * P + row] : 0;
+    float v[PACK_BATCH][5];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b)
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            v[b][j] = j < (int)((uint32_t)w[b] >> RUN_COUNT_SHIFT) ? rvals[(5 * (wv * PACK_BATCH + b) + j) * P + row] : 0.f;
+    const int tot = batch_prefix5(w, ex);
+    if (lane64() == 0) tots[wv] = tot;
+    __syncthreads();
+    for (int u = 0; u < wv; ++u) pos += tots[u];
+#pragma unroll
+    for (int b = 0; b < PACK_BATCH; ++b)
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            if (j < (int)((uint32_t)w[b] >> RUN_COUNT_SHIFT)) pvals[pos + ex[b] + j] = v[b][j];
 }
 
 // Orders a wave's LDS writes before its own later reads (each wave stages into its own region, so
@@ -633,7 +648,7 @@ __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_e
 // 30.2 -> 19.6 at 41k.
 constexpr int64_t WIDE_ROWS = 65536;
 constexpr int WIDE_GROUPS = 2;                        // slices in flight per block
-constexpr int WIDE_WAVES = 25 / PACK_BATCH;           // waves per slice
+constexpr int WIDE_WAVES = PACK_WAVES;                // waves per slice
 constexpr int WIDE_THREADS = 64 * WIDE_WAVES * WIDE_GROUPS;
 
 struct WideLds {
@@ -1719,7 +1734,7 @@ int ngs_runs_pack(const int32_t* runs, const float* rvals, int64_t M, const int6
     if (M <= 0) return NGS_OK;
     NGS_REQUIRE(runs && rvals && soff && pvals, "ngs_runs_pack: null array");
     NGS_REQUIRE(M <= RUN_START_MASK + 1, "ngs_runs_pack: too many rows for run words");
-    runs_pack_kernel<<<grid1d((M + 63) / 64 * 64, PCG_THREADS), PCG_THREADS, 0, S(s)>>>(runs, rvals, M, soff, pvals);
+    runs_pack_kernel<<<grid1d(M, 64), 64 * PACK_WAVES, 0, S(s)>>>(runs, rvals, M, soff, pvals);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }
