@@ -7,6 +7,8 @@
 // and the enlarged pair hash table (jspsr/core/reconstructor.py:71).
 #include "common.h"
 
+#include <algorithm>
+
 namespace ngs {
 
 // Integral tables of one multiple m (device pointers, layout of the reference tables,
@@ -605,63 +607,116 @@ __global__ void rhs_normals_gather_kernel(ngs_level tgt, ngs_level dat, const fl
     rhs[i] += (double)acc;
 }
 
-// Transpose of the field evaluation: out[i] += scale * sum_p w_p B_i(p) over the 27 voxels of g
-// around each point (the adjoint of hashtree.py:157-192).
-__global__ void basis_splat_kernel(ngs_grid g, const float* __restrict__ w, const float* __restrict__ xyz, int64_t n,
-                                   float inv_vs, double scale, double* __restrict__ out) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float wi = w[i];
-    if (wi == 0.f) return;
-    const int s = 1 << g.log2_stride;
-    const float inv_s = 1.0f / (float)s;
-    int cell[3];
-    float b[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) axis_basis(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a]);
-    for (int kx = 0; kx < 3; ++kx)
-        for (int ky = 0; ky < 3; ++ky)
-            for (int kz = 0; kz < 3; ++kz) {
-                int id = grid_find(g, cell[0] + (kx - 1) * s, cell[1] + (ky - 1) * s, cell[2] + (kz - 1) * s);
-                if (id < 0) continue;
-                atomicAdd(&out[id], scale * (double)(wi * (b[0][kx] * b[1][ky] * b[2][kz])));
-            }
-}
+// FP64 sums into a grid's members from many threads. On a coarse grid a few hundred members receive
+// everything and device-scope atomics on one address take turns at the memory side (270k additions into 110
+// members: 143 us), so a block first sums into LDS and adds each of its members once, where the grid fits
+// and that is fewer global atomics than adding directly: `adds` of the whole launch against one per member
+// and block. add() and flush() are called by every thread of the block, flush() once.
+constexpr int MEMBER_LDS = 6144;  // 48 KB
 
-// Transpose of the cross-level stiffness: out_c[j] += scale * sum_i K_{d,dd}(i, j) g_f[i].
-__global__ void cross_stiffness_t_kernel(ngs_level fine, ngs_level coarse, const float* __restrict__ gf, Tables T,
-                                         double scale, double* __restrict__ out) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= fine.M) return;
-    const float gi = gf[i];
-    if (gi == 0.f) return;
-    const int sf_ = fine.stride, sc = coarse.stride, m = T.m;
-    int c[3], Q[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        c[a] = fine.coords[3 * i + a];
-        int num = 2 * c[a] + sf_, den = 2 * sc;
-        int q = num >= 0 ? num / den : -((-num + den - 1) / den);
-        Q[a] = q * sc;
-    }
-    const int nrow = 3 * m + 2;
-    const float fs = (float)sf_, inv_sc = 1.0f / (float)sc;
-    for (int kx = -2; kx <= 2; ++kx) {
-        int ix = kx * m + (Q[0] - c[0]) / sf_ + 2 * m;
-        for (int ky = -2; ky <= 2; ++ky) {
-            int iy = ky * m + (Q[1] - c[1]) / sf_ + 2 * m;
-            for (int kz = -2; kz <= 2; ++kz) {
-                int iz = kz * m + (Q[2] - c[2]) / sf_ + 2 * m;
-                if (ix < 0 || ix >= nrow || iy < 0 || iy >= nrow || iz < 0 || iz >= nrow) continue;
-                int j = grid_find(coarse.grid, Q[0] + kx * sc, Q[1] + ky * sc, Q[2] + kz * sc);
-                if (j < 0) continue;
-                const float c0 = T.F[ix] * fs, c1 = T.F[iy] * fs, c2 = T.F[iz] * fs;
-                const float g0 = T.G[ix] * inv_sc, g1 = T.G[iy] * inv_sc, g2 = T.G[iz] * inv_sc;
-                const float K = g0 * c1 * c2 + c0 * g1 * c2 + c0 * c1 * g2;
-                atomicAdd(&out[j], scale * (double)(K * gi));
-            }
+struct MemberSums {
+    double* lds;
+    double* out;
+    int count;
+    bool local;
+    __device__ __forceinline__ MemberSums(const ngs_grid& g, double* out_, double* lds_, double adds)
+        : lds(lds_), out(out_) {
+        count = as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
+        local = count <= MEMBER_LDS && 2.0 * count * gridDim.x < adds;  // uniform over the grid
+        if (local) {
+            for (int k = threadIdx.x; k < count; k += blockDim.x) lds[k] = 0.0;
+            __syncthreads();
         }
     }
+    __device__ __forceinline__ void add(int id, double v) const {
+        if (local) __hip_atomic_fetch_add(lds + id, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        else atomicAdd(out + id, v);
+    }
+    __device__ __forceinline__ void flush() const {
+        if (!local) return;
+        __syncthreads();
+        for (int k = threadIdx.x; k < count; k += blockDim.x)
+            if (lds[k] != 0.0) atomicAdd(out + k, lds[k]);
+    }
+};
+
+// Blocks for `items` work items of MemberSums kernels: 4 per thread, at most one block per CU.
+static unsigned member_blocks(int64_t items) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, items / 1024)); }
+
+// Transpose of the field evaluation: out[i] += scale * sum_p w_p B_i(p) over the 27 voxels of g
+// around each point (the adjoint of hashtree.py:157-192). One item per (point, bitmap column).
+__global__ void __launch_bounds__(256) basis_splat_kernel(ngs_grid g, const float* __restrict__ w,
+                                                          const float* __restrict__ xyz, int64_t n, float inv_vs,
+                                                          double scale, double* __restrict__ out) {
+    __shared__ double lds[MEMBER_LDS];
+    const MemberSums sums(g, out, lds, 27.0 * n);
+    const int s = 1 << g.log2_stride, l2 = g.log2_stride;
+    const float inv_s = 1.0f / (float)s;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 9 * n; t += (int64_t)gridDim.x * 256) {
+        const int64_t i = t / 9;
+        const int col = (int)(t - 9 * i), kx = col / 3, ky = col % 3;
+        const float wi = w[i];
+        if (wi == 0.f) continue;
+        int cell[3];
+        float b[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) axis_basis(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a]);
+        int32_t id = 0;
+        const uint32_t m = grid_column(g, (cell[0] >> l2) - g.origin[0] + kx - 1, (cell[1] >> l2) - g.origin[1] + ky - 1,
+                                       (cell[2] >> l2) - g.origin[2] - 1, 3, &id);
+        const float bx = kx == 0 ? b[0][0] : kx == 1 ? b[0][1] : b[0][2];
+        const float by = ky == 0 ? b[1][0] : ky == 1 ? b[1][1] : b[1][2];
+#pragma unroll
+        for (int kz = 0; kz < 3; ++kz)
+            if ((m >> kz) & 1u) sums.add(id++, scale * (double)(wi * (bx * by * b[2][kz])));
+    }
+    sums.flush();
+}
+
+// Transpose of the cross-level stiffness: out_c[j] += scale * sum_i K_{d,dd}(i, j) g_f[i]. One item per (fine
+// voxel, coarse bitmap column).
+__global__ void __launch_bounds__(256) cross_stiffness_t_kernel(ngs_level fine, ngs_level coarse,
+                                                                const float* __restrict__ gf, Tables T, double scale,
+                                                                double* __restrict__ out) {
+    __shared__ double lds[MEMBER_LDS];
+    const MemberSums sums(coarse.grid, out, lds, 60.0 * fine.M);
+    const int sf_ = fine.stride, sc = coarse.stride, m = T.m;
+    const int nrow = 3 * m + 2;
+    const float fs = (float)sf_, inv_sc = 1.0f / (float)sc;
+    const ngs_grid& g = coarse.grid;
+    const int l2 = g.log2_stride;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 25 * fine.M; t += (int64_t)gridDim.x * 256) {
+        const int64_t i = t / 25;
+        const int col = (int)(t - 25 * i), kx = col / 5 - 2, ky = col % 5 - 2;
+        const float gi = gf[i];
+        if (gi == 0.f) continue;
+        int c[3], Q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            c[a] = fine.coords[3 * i + a];
+            int num = 2 * c[a] + sf_, den = 2 * sc;
+            int q = num >= 0 ? num / den : -((-num + den - 1) / den);
+            Q[a] = q * sc;
+        }
+        const int ix = kx * m + (Q[0] - c[0]) / sf_ + 2 * m, iy = ky * m + (Q[1] - c[1]) / sf_ + 2 * m;
+        if (ix < 0 || ix >= nrow || iy < 0 || iy >= nrow) continue;
+        int32_t id = 0;
+        const uint32_t mask = grid_column(g, (Q[0] >> l2) - g.origin[0] + kx, (Q[1] >> l2) - g.origin[1] + ky,
+                                          (Q[2] >> l2) - g.origin[2] - 2, 5, &id);
+        if (!mask) continue;
+        const float c0 = T.F[ix] * fs, c1 = T.F[iy] * fs, g0 = T.G[ix] * inv_sc, g1 = T.G[iy] * inv_sc;
+#pragma unroll
+        for (int kz = -2; kz <= 2; ++kz) {
+            if (!((mask >> (kz + 2)) & 1u)) continue;
+            const int j = id++;
+            const int iz = kz * m + (Q[2] - c[2]) / sf_ + 2 * m;
+            if (iz < 0 || iz >= nrow) continue;
+            const float c2 = T.F[iz] * fs, g2 = T.G[iz] * inv_sc;
+            const float K = g0 * c1 * c2 + c0 * g1 * c2 + c0 * c1 * g2;
+            sums.add(j, scale * (double)(K * gi));
+        }
+    }
+    sums.flush();
 }
 
 }  // namespace ngs
@@ -883,7 +938,7 @@ int ngs_rhs_normals(ngs_level target, ngs_level data, const float* normals, doub
 int ngs_basis_splat(ngs_grid g, const float* w, const float* xyz, int64_t n, float inv_voxel_size, double scale, double* out,
                     ngs_stream_t s) {
     if (n <= 0) return NGS_OK;
-    basis_splat_kernel<<<grid1d(n, 256), 256, 0, S(s)>>>(g, w, xyz, n, inv_voxel_size, scale, out);
+    basis_splat_kernel<<<member_blocks(9 * n), 256, 0, S(s)>>>(g, w, xyz, n, inv_voxel_size, scale, out);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }
@@ -894,7 +949,7 @@ int ngs_cross_stiffness_transpose(ngs_level fine, ngs_level coarse, const float*
     NGS_REQUIRE(coarse.stride > fine.stride, "ngs_cross_stiffness_transpose: coarse stride must exceed fine stride");
     Tables T;
     NGS_REQUIRE(tables_for(coarse.stride / fine.stride, &T), "ngs_cross_stiffness_transpose: table multiple unavailable");
-    cross_stiffness_t_kernel<<<grid1d(fine.M, 128), 128, 0, S(s)>>>(fine, coarse, g_fine, T, scale, out_coarse);
+    cross_stiffness_t_kernel<<<member_blocks(25 * fine.M), 256, 0, S(s)>>>(fine, coarse, g_fine, T, scale, out_coarse);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }

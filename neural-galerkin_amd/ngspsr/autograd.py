@@ -98,8 +98,9 @@ class DifferentiableScreenedPoisson:
                 g_scale[d] = torch.zeros(0, dtype=torch.float64, device=tree.device)
                 continue
             sf = 0.25 ** d
+            filt = _solver.system_filter(self.systems[d])
             g_b, _ = _solver.pcg(self.systems[d], g_x[d].float(), tol=self.adjoint_tol, maxiter=50000,
-                                 raise_on_cap=False)
+                                 chunk=32 if filt is None else _solver.FILTER_CHUNK, raise_on_cap=False, filt=filt)
             g_scale[d] = g_b.double() * self.n_rhs[d]
             G = torch.zeros(n, dtype=torch.float32, device=tree.device)
             self._field_at_points(d, g_b, G, accumulate=False)
