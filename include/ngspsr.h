@@ -179,6 +179,9 @@ int ngs_splat_gather(ngs_grid g, const int32_t *node_coords, int64_t count, cons
  * the derivative with respect to q (finest-voxel units), as evaluate_derivative returns it. */
 int ngs_eval_field(ngs_grid g, const float *field, const float *xyz, int64_t n, float inv_voxel_size,
                    float scale, int32_t accumulate, float *out, float *grad_out, ngs_stream_t s);
+/* counts[l] = points of level l, l < depth (at most 4096), counts[depth] = points of other levels
+ * (depth + 1 int64). */
+int ngs_level_counts(const int32_t *levels, int64_t n, int32_t depth, int64_t *counts, ngs_stream_t s);
 /* ngs_eval_field without gradient, queries processed in the order of the permutation `order` (n int32): the
  * same values (out stays in query order), faster when `order` brings neighbouring queries together. */
 int ngs_eval_field_ordered(ngs_grid g, const float *field, const float *xyz, const int32_t *order, int64_t n,

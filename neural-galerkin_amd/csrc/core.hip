@@ -1,6 +1,7 @@
 // Keys, cuckoo table, ordered bitmap sets, scans, density/levels, splat and field evaluation.
 #include "common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #include <cmath>
@@ -833,6 +834,25 @@ __global__ void levels_kernel(const float* __restrict__ rho, int64_t n, float in
     lv[i] = k;
 }
 
+// counts[l] += points of level l < depth, counts[depth] += the others (counts zeroed before).
+__global__ void __launch_bounds__(256) level_counts_kernel(const int32_t* __restrict__ levels, int64_t n, int depth,
+                                                           unsigned long long* __restrict__ counts) {
+    extern __shared__ unsigned int hist[];
+    for (int k = threadIdx.x; k <= depth; k += 256) hist[k] = 0;
+    __syncthreads();
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int l = levels[i], b = (unsigned)l < (unsigned)depth ? l : depth;
+        // most points share a level: one addition for the lanes of the first lane's level
+        const int first = __builtin_amdgcn_readfirstlane(b);
+        const uint64_t same = __ballot(b == first);
+        if (b != first) atomicAdd(&hist[b], 1u);
+        else if (lane64() == __ffsll((unsigned long long)same) - 1) atomicAdd(&hist[b], (unsigned)__popcll(same));
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k <= depth; k += 256)
+        if (hist[k]) atomicAdd(&counts[k], (unsigned long long)hist[k]);
+}
+
 __global__ void point_basis_kernel(const float* __restrict__ xyz, int64_t n, float inv_vs, int s,
                                    int32_t* __restrict__ cell, float* __restrict__ b) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1288,6 +1308,16 @@ int ngs_eval_field_ordered(ngs_grid g, const float* field, const float* xyz, con
     NGS_REQUIRE(xyz && order && out, "ngs_eval_field_ordered: null argument");
     eval_field_kernel<false><<<grid1d(n, 256), 256, 0, S(s)>>>(g, field, xyz, order, n, inv_voxel_size, scale,
                                                                accumulate, out, nullptr);
+    NGS_CHECK_LAUNCH();
+    return NGS_OK;
+}
+
+int ngs_level_counts(const int32_t* levels, int64_t n, int32_t depth, int64_t* counts, ngs_stream_t s) {
+    NGS_REQUIRE(depth >= 1 && depth <= 4096 && counts && (levels || n <= 0), "ngs_level_counts: bad arguments");
+    zero_i32<<<grid1d(2 * (depth + 1), 256), 256, 0, S(s)>>>(reinterpret_cast<int32_t*>(counts), 2 * (depth + 1));
+    if (n > 0)
+        level_counts_kernel<<<(unsigned)std::min<int64_t>(1024, (n + 255) / 256), 256, sizeof(unsigned) * (depth + 1),
+                              S(s)>>>(levels, n, depth, reinterpret_cast<unsigned long long*>(counts));
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }

@@ -78,6 +78,7 @@ _SIGNATURES = {
     "ngs_splat_gather_workspace_bytes": ([c_int64, c_int64], c_int64),
     "ngs_splat_gather": ([Grid, P, c_int64, P, c_int64, c_float, P, c_int32, P, P, c_int32, c_double, P, P, c_int64, P],
                          c_int32),
+    "ngs_level_counts": ([P, c_int64, c_int32, P, P], c_int32),
     "ngs_eval_field_ordered": ([Grid, P, P, P, c_int64, c_float, c_float, c_int32, P, P], c_int32),
     "ngs_splat_gather_order_offset": ([c_int64, c_int64], c_int64),
     "ngs_eval_field": ([Grid, P, P, c_int64, c_float, c_float, c_int32, P, P, P], c_int32),

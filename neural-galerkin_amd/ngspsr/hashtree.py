@@ -330,6 +330,19 @@ class HashTree:
             grids.append(g)
         return SparseGrid.finalize_all(grids)
 
+    def _count_levels(self, lv):
+        """Points per level, as torch.bincount(lv, minlength=depth) gives them (one pass, one read; its
+        own pass where imposed levels leave the range: longer counts, or its error for negative ones)."""
+        n, depth = lv.shape[0], self._depth
+        if lv.dim() != 1 or depth > 4096:
+            return torch.bincount(lv.long(), minlength=depth).cpu().numpy()
+        counts = torch.empty(depth + 1, dtype=torch.int64, device=self.device)
+        call("ngs_level_counts", ptr(lv), n, depth, ptr(counts), stream())
+        c = counts.cpu().numpy()
+        if c[depth]:
+            return torch.bincount(lv.long(), minlength=depth).cpu().numpy()
+        return c[:depth]
+
     def build_encoder_hierarchy_adaptive(self, density_depth: int = 2, log_base: float = 4.0, min_density: float = 8.0,
                                          uniform_density: bool = False, limit_adaptive_depth: int = 100,
                                          xyz_depth=None):
@@ -347,7 +360,7 @@ class HashTree:
         else:
             lv = xyz_depth.to(device=self.device, dtype=torch.int32).contiguous()
         self.xyz_depth = lv
-        self._level_counts = torch.bincount(lv.long(), minlength=self._depth).cpu().numpy()
+        self._level_counts = self._count_levels(lv)
         self._set_encoder_levels(self._corner_levels(lv))
         return self.xyz_depth
 
@@ -423,7 +436,7 @@ class HashTree:
             grids[d] = g
         xyz_depth.clamp_(max=limit_adaptive_depth - 1)
         self.xyz_depth = xyz_depth
-        self._level_counts = torch.bincount(xyz_depth.long(), minlength=self._depth).cpu().numpy()
+        self._level_counts = self._count_levels(xyz_depth)
         if expand:
             grids = self._corner_levels(xyz_depth)
         else:
