@@ -243,6 +243,17 @@ __device__ __forceinline__ T run_row_dot(const NGS_GLOBAL int32_t* __restrict__ 
     return sum;
 }
 
+// Which of the matrix streams of a packed system of M rows bypass the caches (non-temporal loads): once the
+// matrix no longer fits the last-level cache (256 MB, ~550k rows of ~465 bytes) every product sweeps the
+// vectors of the other steps out of it. Values only from 650k rows, the run words too from 2.7M (below,
+// their lines are shared by the slices around them). Measured, us per filtered iteration with plain loads /
+// values / both: 261k rows 45.5 48.8 48.8, 525k 63.2 70.8 74.4, 884k 131 119 128, 1.14M 169 150 161, 2.17M 226 222
+// 212 (Jacobi 187 166 184), 3.18M 350 350 331, 4.26M 514 519 490 (Jacobi 444 451 440), 5.6M 715 727 712.
+constexpr int STREAM_VALUES = 1, STREAM_RUNS = 2;
+__host__ __device__ __forceinline__ int packed_streams(int64_t M) {
+    return M > 2700000 ? STREAM_VALUES | STREAM_RUNS : M > 650000 ? STREAM_VALUES : 0;
+}
+
 // ---------------------------------------------------------------------- filtered preconditioner
 // The level matrices are sums of B-spline mass and stiffness terms, whose eigenvalues at the lattice's
 // highest frequencies are far below those in the middle of the spectrum (per axis the mass symbol falls
@@ -281,10 +292,11 @@ __device__ __forceinline__ float filter_scale(float dinv) { return sqrtf(fabsf(d
 // column (0, 0) holds the row itself.
 __device__ __forceinline__ float filter_row(const NGS_GLOBAL int32_t* __restrict__ words,
                                             const NGS_GLOBAL float* __restrict__ s, int64_t P, int64_t row, float w1,
-                                            float w2, float w3) {
+                                            float w2, float w3, bool stream) {
     uint32_t w[FILTER_COLS];
 #pragma unroll
-    for (int c = 0; c < FILTER_COLS; ++c) w[c] = (uint32_t)words[c * P + row];
+    for (int c = 0; c < FILTER_COLS; ++c) w[c] = (uint32_t)(stream ? __builtin_nontemporal_load(words + c * P + row)
+                                                                    : words[c * P + row]);
     float v[FILTER_COLS][3];
 #pragma unroll
     for (int c = 0; c < FILTER_COLS; ++c) {
@@ -314,10 +326,11 @@ __device__ __forceinline__ void filter_rows(const PcgArgs& A, float* out, int lb
     const NGS_GLOBAL float* __restrict__ dinv = as_global(A.dinv);
     NGS_GLOBAL float* __restrict__ z = as_global(out);
     const float w1 = A.fw[0], w2 = A.fw[1], w3 = A.fw[2];
+    const bool stream = packed_streams(A.M) != 0;  // as the matrix
     double rz = 0;
     for (int64_t i = r0 + threadIdx.x; i < r1; i += PCG_THREADS) {
         const float si = s[i], di = dinv[i];
-        const float g = filter_row(words, s, P, i, w1, w2, w3);
+        const float g = filter_row(words, s, P, i, w1, w2, w3, stream);
         z[i] = filter_scale(di) * g;
         rz += (double)si * g;
     }
@@ -548,6 +561,20 @@ __global__ void __launch_bounds__(64 * PACK_WAVES) runs_pack_kernel(const int32_
             if (j < (int)((uint32_t)w[b] >> RUN_COUNT_SHIFT)) pvals[pos + ex[b] + j] = v[b][j];
 }
 
+// f(integral_constant of packed_streams(M)).
+template <class F>
+__host__ __device__ __forceinline__ void with_streams(int64_t M, F&& f) {
+    const int st = packed_streams(M);
+    if (st == 0) f(std::integral_constant<int, 0>());
+    else if (st == STREAM_VALUES) f(std::integral_constant<int, STREAM_VALUES>());
+    else f(std::integral_constant<int, STREAM_VALUES | STREAM_RUNS>());
+}
+
+template <bool STREAM, typename T>
+__device__ __forceinline__ T load_once(const NGS_GLOBAL T* p) {
+    return STREAM ? __builtin_nontemporal_load(p) : *p;
+}
+
 // Orders a wave's LDS writes before its own later reads (each wave stages into its own region, so
 // the block's waves need not wait for each other).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -561,7 +588,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // the wave stages the batch's values (contiguous in pvals) into its LDS region with coalesced loads,
 // then every lane reads its runs there and gathers x. Each wave has its own LDS region, ordered by
 // wave-scope fences; lanes past M carry empty runs.
-template <typename T, typename XT>
+// STREAMS: packed_streams.
+template <typename T, typename XT, int STREAMS>
 __device__ __forceinline__ T packed_row_dot(const NGS_GLOBAL int32_t* __restrict__ runs,
                                             const NGS_GLOBAL float* __restrict__ pvals,
                                             const NGS_GLOBAL XT* __restrict__ x, int64_t P, int64_t row, bool ok,
@@ -573,7 +601,7 @@ __device__ __forceinline__ T packed_row_dot(const NGS_GLOBAL int32_t* __restrict
         int32_t w[PACK_BATCH];
         int ex[PACK_BATCH];
 #pragma unroll
-        for (int b = 0; b < PACK_BATCH; ++b) w[b] = ok ? runs[(p0 + b) * P + row] : 0;
+        for (int b = 0; b < PACK_BATCH; ++b) w[b] = ok ? load_once<(STREAMS & STREAM_RUNS) != 0>(runs + (p0 + b) * P + row) : 0;
         const int tot = batch_prefix5(w, ex);
         {
             // all of the batch's loads issued together (one memory round trip per batch): lane l takes
@@ -582,7 +610,7 @@ __device__ __forceinline__ T packed_row_dot(const NGS_GLOBAL int32_t* __restrict
 #pragma unroll
             for (int u = 0; u < PACK_STAGE / 64; ++u) {
                 const int e = u * 64 + lane;
-                t[u] = (u * 64 < tot && e < tot) ? pvals[pos + e] : 0.f;
+                t[u] = (u * 64 < tot && e < tot) ? load_once<(STREAMS & STREAM_VALUES) != 0>(pvals + pos + e) : 0.f;
             }
 #pragma unroll
             for (int u = 0; u < PACK_STAGE / 64; ++u) {
@@ -615,6 +643,7 @@ __device__ __forceinline__ T packed_row_dot(const NGS_GLOBAL int32_t* __restrict
 
 // y = A x for the packed form: blocks of 4 waves take groups of 4 slices, grid-stride. Capped at 5 waves
 // per SIMD; with the scan-based run prefixes it needs 80 VGPRs, so the LDS (6 blocks per CU) sets 6.
+template <int STREAMS>
 __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_eu(5))) spmv_packed_kernel(const int32_t* __restrict__ runs,
                                                                   const float* __restrict__ pvals,
                                                                   const int64_t* __restrict__ soff,
@@ -631,8 +660,8 @@ __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_e
         const int64_t row = sl * 64 + lane64();
         const bool ok = row < M;
         const int64_t pos = sl < nsl ? soff[sl] : 0;
-        const float sum = packed_row_dot<float, float>(as_global(runs), as_global(pvals), as_global(x), P, row, ok,
-                                                       pos, stage);
+        const float sum = packed_row_dot<float, float, STREAMS>(as_global(runs), as_global(pvals), as_global(x), P,
+                                                                row, ok, pos, stage);
         if (ok) y[row] = sum;
     }
 }
@@ -828,6 +857,7 @@ __global__ void __launch_bounds__(PCG_THREADS) residual_f64_runs_kernel(const in
 // take 256-row groups (4 slices), grid-stride. The norms are summed by norms2_kernel afterwards: with
 // its FP64 accumulators the row loop here would hold 2 waves per SIMD instead of 3 (172 VGPRs), and a
 // separate pass over r and b (16 bytes per row) costs less than the lost occupancy.
+template <int STREAMS>
 __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 residual_f64_packed_kernel(const int32_t* __restrict__ runs, const float* __restrict__ pvals,
                            const int64_t* __restrict__ soff, const double* __restrict__ b,
@@ -842,8 +872,8 @@ residual_f64_packed_kernel(const int32_t* __restrict__ runs, const float* __rest
         const bool ok = row < M;
         const int64_t sl = row >> 6;
         const int64_t pos = sl < nsl ? soff[sl] : 0;
-        const double ax = x ? packed_row_dot<double, double>(as_global(runs), as_global(pvals), as_global(x), P, row,
-                                                             ok, pos, stage)
+        const double ax = x ? packed_row_dot<double, double, STREAMS>(as_global(runs), as_global(pvals), as_global(x),
+                                                                      P, row, ok, pos, stage)
                             : 0.0;
         if (ok) r[row] = x ? b[row] - ax : b[row];
     }
@@ -1111,19 +1141,22 @@ __global__ void __launch_bounds__(PCG_THREADS) __attribute__((amdgpu_waves_per_e
     const NGS_GLOBAL float* __restrict__ p = as_global(A.p);
     NGS_GLOBAL float* __restrict__ q = as_global(A.q);
     double pq = 0;
-    for (int64_t base = (int64_t)(blockIdx.x - B->blk0) * PCG_THREADS; base < A.M; base += step) {
-        const int64_t row = base + threadIdx.x;
-        const bool ok = row < A.M;
-        const int64_t sl = row >> 6;
-        const int64_t pos = sl < nsl ? A.soff[sl] : 0;
-        const float prow = ok ? p[row] : 0.f;
-        const float sum = packed_row_dot<float, float>(as_global(A.runs), as_global(A.rvals), p, P, row, ok, pos,
-                                                       stage);
-        if (ok) {
-            q[row] = sum;
-            pq += (double)prow * sum;
+    auto rows = [&](auto streams) {
+        for (int64_t base = (int64_t)(blockIdx.x - B->blk0) * PCG_THREADS; base < A.M; base += step) {
+            const int64_t row = base + threadIdx.x;
+            const bool ok = row < A.M;
+            const int64_t sl = row >> 6;
+            const int64_t pos = sl < nsl ? A.soff[sl] : 0;
+            const float prow = ok ? p[row] : 0.f;
+            const float sum = packed_row_dot<float, float, decltype(streams)::value>(
+                as_global(A.runs), as_global(A.rvals), p, P, row, ok, pos, stage);
+            if (ok) {
+                q[row] = sum;
+                pq += (double)prow * sum;
+            }
         }
-    }
+    };
+    with_streams(A.M, rows);
     store_partials2(pq, 0.0, A.partials, nullptr, lb);
 }
 
@@ -1759,7 +1792,9 @@ int ngs_spmv_packed(const int32_t* runs, const float* pvals, const int64_t* soff
     if (M <= WIDE_ROWS)
         spmv_packed_wide_kernel<<<grid1d(M, 64 * WIDE_GROUPS), WIDE_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
     else
-        spmv_packed_kernel<<<nb, PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
+        with_streams(M, [&](auto streams) {
+            spmv_packed_kernel<decltype(streams)::value><<<nb, PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, x, y, M);
+        });
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }
@@ -1826,8 +1861,10 @@ int ngs_residual_f64_packed(const int32_t* runs, const float* pvals, const int64
     char* w = reinterpret_cast<char*>(workspace);
     double* partials = reinterpret_cast<double*>(w + al256(sizeof(PcgState)));
     const int64_t groups = ((M + 63) / 64 + 3) / 4;
-    residual_f64_packed_kernel<<<(int)std::min<int64_t>(groups, 8192), PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, b, x,
-                                                                                               r, M);
+    with_streams(M, [&](auto streams) {
+        residual_f64_packed_kernel<decltype(streams)::value>
+            <<<(int)std::min<int64_t>(groups, 8192), PCG_THREADS, 0, S(s)>>>(runs, pvals, soff, b, x, r, M);
+    });
     norms2_kernel<<<nb, PCG_THREADS, 0, S(s)>>>(r, b, M, chunk, partials);
     norms_finish_kernel<<<1, PCG_THREADS, 0, S(s)>>>(partials, nb, norms);
     NGS_CHECK_LAUNCH();
