@@ -599,6 +599,17 @@ int ngs_mark_dual_leaf_words(ngs_grid centres, ngs_grid leaf_bitmap, ngs_stream_
 int ngs_dual_gather_cubes(const int32_t *centre_coords, int64_t dc, int32_t nlevels, const ngs_grid *leaf_bitmaps,
                           const int32_t *const *leaf_index, const int32_t *id_base, const float *values, int32_t *acc,
                           int32_t *count, ngs_stream_t s);
+/* The cubes with triangles only, as ngs_dual_gather_cubes followed by ngs_dual_compact (active_only)
+ * would leave them: rows (dc x 8) receives them packed at the start of each block of centres,
+ * block_counts (ngs_dual_active_blocks(dc)) how many each block has; ngs_dual_compact_active moves
+ * them together in centre order (cubes, at most dc x 8), block_offsets (blocks + 1) ending with their
+ * number; workspace: ngs_scan_workspace_bytes(blocks). */
+int64_t ngs_dual_active_blocks(int64_t dc);
+int ngs_dual_gather_active(const int32_t *centre_coords, int64_t dc, int32_t nlevels, const ngs_grid *leaf_bitmaps,
+                           const int32_t *const *leaf_index, const int32_t *id_base, const float *values, int32_t *rows,
+                           int32_t *block_counts, ngs_stream_t s);
+int ngs_dual_compact_active(const int32_t *rows, const int32_t *block_counts, int64_t dc, int32_t *block_offsets,
+                            int32_t *cubes, void *workspace, ngs_stream_t s);
 int ngs_dual_accumulate_leaves(ngs_grid centres, const int32_t *leaves, int64_t n, int32_t n_upsample,
                                int32_t id_base, const float *values, int32_t *acc, int32_t *count, ngs_stream_t s);
 /* Dual-corner positions (primal + stride) * voxel_size / n_upsample (reconstructor.py:368-373). */

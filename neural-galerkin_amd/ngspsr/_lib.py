@@ -163,6 +163,9 @@ _SIGNATURES = {
     "ngs_mark_dual_leaves": ([Grid, P, c_int64, c_int32, c_int32, P], c_int32),
     "ngs_mark_dual_leaf_words": ([Grid, Grid, P], c_int32),
     "ngs_dual_gather_cubes": ([P, c_int64, c_int32, P, P, P, P, P, P, P], c_int32),
+    "ngs_dual_active_blocks": ([c_int64], c_int64),
+    "ngs_dual_gather_active": ([P, c_int64, c_int32, P, P, P, P, P, P, P], c_int32),
+    "ngs_dual_compact_active": ([P, P, c_int64, P, P, P, P], c_int32),
     "ngs_dual_accumulate_leaves": ([Grid, P, c_int64, c_int32, c_int32, P, P, P, P], c_int32),
     "ngs_dual_compact": ([P, P, c_int32, c_int64, P, P, P, P, P], c_int32),
     "ngs_dual_corner_positions": ([P, c_int64, c_int32, c_float, P, P], c_int32),

@@ -703,6 +703,7 @@ class Reconstructor:
                 call("ngs_mark_dual_leaves", cg.struct(), ptr(leaves[d]), leaves[d].shape[0], tree.strides[d], nu,
                      stream())
         DC = cg.finalize(emit=return_info or gather)  # coordinates read by the gathered assembly
+        active = gather and not return_info  # without the report only the cubes with triangles are needed
         # dual corners = (primal + stride) * voxel_size / n_upsample, and chi there
         pos = torch.empty((nprim, 3), dtype=torch.float32, device=dev)
         scale = float(np.float32(tree.voxel_size / nu))
@@ -717,7 +718,8 @@ class Reconstructor:
         # primal id per octant, read only for the kept centres (all eight slots written); the count
         # word also counts the registered cells with a negative value
         acc = torch.empty((DC, 8), dtype=torch.int32, device=dev)
-        cnt = torch.zeros(DC, dtype=torch.int32, device=dev)
+        cnt = None if active else torch.zeros(DC, dtype=torch.int32, device=dev)
+        blocks = lib().ngs_dual_active_blocks(DC) if active else 0
         if gather:
             # n_upsample 2: every level's cubes gathered per centre from per-level leaf bitmaps (no atomics)
             bitmaps, index, base = [], [], []
@@ -742,8 +744,13 @@ class Reconstructor:
                 garr = (Grid * nl)(*[g.struct() for g in bitmaps])
                 iarr = (ctypes.c_void_p * nl)(*[t.data_ptr() for t in index])
                 barr = (ctypes.c_int32 * nl)(*base)
-                call("ngs_dual_gather_cubes", ptr(cg.coords), DC, nl, garr, iarr, barr, ptr(values), ptr(acc),
-                     ptr(cnt), stream())
+                if active:
+                    cnt = torch.empty(blocks, dtype=torch.int32, device=dev)
+                    call("ngs_dual_gather_active", ptr(cg.coords), DC, nl, garr, iarr, barr, ptr(values), ptr(acc),
+                         ptr(cnt), stream())
+                else:
+                    call("ngs_dual_gather_cubes", ptr(cg.coords), DC, nl, garr, iarr, barr, ptr(values), ptr(acc),
+                         ptr(cnt), stream())
         else:
             for d in range(L):
                 if not nsub[d]:
@@ -756,11 +763,18 @@ class Reconstructor:
                          bases_[d], ptr(values), ptr(acc), ptr(cnt), stream())
         # complete cubes whose corner values change sign (the only ones with triangles), in centre order
         cubes = torch.empty((DC, 8), dtype=torch.int32, device=dev)
-        flags = torch.empty(DC, dtype=torch.int32, device=dev)
-        offs = torch.empty(DC + 1, dtype=torch.int32, device=dev)
-        ws = Scratch.get(lib().ngs_scan_workspace_bytes(DC), dev)
-        call("ngs_dual_compact", ptr(acc), ptr(cnt), 1, DC, ptr(cubes), ptr(flags), ptr(offs), ptr(ws), stream())
-        K = int(offs[DC].item()) if DC else 0
+        n = blocks if active else DC
+        if cnt is None or DC == 0:
+            K = 0
+        else:
+            offs = torch.empty(n + 1, dtype=torch.int32, device=dev)
+            ws = Scratch.get(lib().ngs_scan_workspace_bytes(n), dev)
+            if active:
+                call("ngs_dual_compact_active", ptr(acc), ptr(cnt), DC, ptr(offs), ptr(cubes), ptr(ws), stream())
+            else:
+                flags = torch.empty(DC, dtype=torch.int32, device=dev)
+                call("ngs_dual_compact", ptr(acc), ptr(cnt), 1, DC, ptr(cubes), ptr(flags), ptr(offs), ptr(ws), stream())
+            K = int(offs[n].item())
         cubes = cubes[:K]
         v, f = self.dual_marching_cubes(cubes, pos, values)
         if return_info:
