@@ -133,6 +133,11 @@ __device__ __forceinline__ uint32_t grid_column(const ngs_grid& g, int lx, int l
     return m << (zlo - lz0);
 }
 
+// Members of g (its last rank).
+__device__ __forceinline__ int32_t grid_count(const ngs_grid& g) {
+    return as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
+}
+
 __device__ __forceinline__ int lane64() { return (int)(threadIdx.x & 63); }
 
 // Logical index of this block such that the blocks of each XCD form one contiguous range. Blocks are

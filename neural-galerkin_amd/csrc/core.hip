@@ -671,11 +671,6 @@ __global__ void __launch_bounds__(256) splat_gather_kernel(ngs_grid g, const int
     }
 }
 
-// Members of g (its last rank).
-__device__ __forceinline__ int32_t grid_count(const ngs_grid& g) {
-    return as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
-}
-
 // Coefficients of the three columns (lx, ly - 1 .. ly + 1, lz - 1 .. lz + 1) around a cell, 0 where absent:
 // the columns' bitmap words together, then their ranks, then one 12-byte load per column (its present
 // voxels have consecutive ranks). Three waits for three columns instead of two for each, and a third of the
