@@ -26,14 +26,11 @@ import torch
 from . import _lib
 from ._lib import NgsError, call, lib, ptr, stream
 
-DEFAULTS = {"pcg": {"tol": 1e-5, "maxiter": -1, "res_fix": False, "verbose": False, "chunk": 16},
-            "mixed": {"tol": 1e-2, "fast_tol": 1e-4, "fast_maxiter": 1000, "verbose": False, "chunk": 16},
-            "cholmod": {"tol": 1e-6, "verbose": False, "chunk": 16},
+DEFAULTS = {"pcg": {"tol": 1e-5, "maxiter": -1, "res_fix": False, "verbose": False, "chunk": 32},
+            "mixed": {"tol": 1e-2, "fast_tol": 1e-4, "fast_maxiter": 1000, "verbose": False, "chunk": 32},
+            "cholmod": {"tol": 1e-6, "verbose": False, "chunk": 32},
             "refine": {"tol": 1e-8, "maxiter": 100000, "inner_tol": 1e-4, "max_outer": 20, "verbose": False,
-                       "chunk": 16}}
-# chunk: iterations per launch sequence. A sequence costs a host read (~25 us), and the iterations left in
-# it when the solve ends cost their empty launches (6 us each on small systems, 13 at 2560 blocks): for
-# 30-50 iterations 12 to 18 per sequence are best.
+                       "chunk": 32}}
 
 
 def parse_solver(spec: str):
