@@ -32,6 +32,12 @@ DEFAULTS = {"pcg": {"tol": 1e-5, "maxiter": -1, "res_fix": False, "verbose": Fal
             "refine": {"tol": 1e-8, "maxiter": 100000, "inner_tol": 1e-4, "max_outer": 20, "verbose": False,
                        "chunk": 32}}
 
+# Iterations per launch sequence of a solver string that names no chunk. A sequence costs a
+# host read (~25 us), and the iterations left in it when the solve ends cost their empty launches (6 us each on
+# small systems, 13 at 2560 blocks): for 14-50 iterations 12 to 18 per sequence are best (20k-point
+# reconstruction 3.58 ms at 32, 3.30 at 16).
+PCG_CHUNK = 16
+
 
 def parse_solver(spec: str):
     parts = spec.split("@")
@@ -607,18 +613,19 @@ def solve(system, b, spec: str = "pcg"):
     (the refinement's FP64 iterate, whose residual SolveInfo.rel_resid reports) and "cholmod" (the
     FP64 direct solution)."""
     name, conf = parse_solver(spec)
+    chunk = conf["chunk"] if "@chunk=" in spec else PCG_CHUNK
     if name == "pcg":
-        x, info = pcg(system, b, tol=conf["tol"], maxiter=conf["maxiter"], chunk=conf["chunk"])
+        x, info = pcg(system, b, tol=conf["tol"], maxiter=conf["maxiter"], chunk=chunk)
     elif name == "mixed":
         x, info = mixed(system, b, tol=conf["tol"], fast_tol=conf["fast_tol"], fast_maxiter=conf["fast_maxiter"],
-                        chunk=conf["chunk"])
+                        chunk=chunk)
     elif name == "cholmod":
-        x, info = cholmod(system, b, tol=conf["tol"], chunk=conf["chunk"])
+        x, info = cholmod(system, b, tol=conf["tol"], chunk=chunk)
     else:
         # the FP64 iterate is the solution: its FP64 residual is the one SolveInfo reports (its FP32
         # rounding would sit at the FP32 floor, ~1e-8 relative, above the tighter tolerances)
         x, info = refine(system, b, tol=conf["tol"], inner_tol=conf["inner_tol"], max_outer=conf["max_outer"],
-                         maxiter=conf["maxiter"], chunk=conf["chunk"])
+                         maxiter=conf["maxiter"], chunk=chunk)
     if conf.get("verbose"):
         print("PCG Iteration ended in", info.iters)
     return x, info
