@@ -621,7 +621,7 @@ struct MemberSums {
     bool local;
     __device__ __forceinline__ MemberSums(const ngs_grid& g, double* out_, double* lds_, double adds)
         : lds(lds_), out(out_) {
-        count = as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
+        count = grid_count(g);
         local = count <= MEMBER_LDS && 2.0 * count * gridDim.x < adds;  // uniform over the grid
         if (local) {
             for (int k = threadIdx.x; k < count; k += blockDim.x) lds[k] = 0.0;

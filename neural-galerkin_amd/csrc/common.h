@@ -133,8 +133,9 @@ __device__ __forceinline__ uint32_t grid_column(const ngs_grid& g, int lx, int l
     return m << (zlo - lz0);
 }
 
-// Members of g (its last rank).
+// Members of g (its last rank). A grid without words (all fields 0, no buffers) has none and is not read.
 __device__ __forceinline__ int32_t grid_count(const ngs_grid& g) {
+    if (g.nwords <= 0) return 0;
     return as_global(g.rank)[g.nwords - 1] + __popc(as_global(g.bits)[g.nwords - 1]);
 }
 

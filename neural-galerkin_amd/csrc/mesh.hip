@@ -276,7 +276,7 @@ __device__ __forceinline__ void eval_leaf_corners_one(const ngs_grid& g, const f
     if (nu == 2) {
         int cell[3][2];
         float b[3][2][3];
-        bool window = g.nwords > 0 && grid_count(g) > 0;
+        bool window = grid_count(g) > 0;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const int p = lf[a] * 2;
