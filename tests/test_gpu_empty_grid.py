@@ -29,7 +29,7 @@ def test_field_and_its_transpose_on_a_grid_without_words(cuda, n):
     cell = torch.zeros((n, 3), dtype=torch.int32, device=cuda)
     basis = torch.rand(n, 9, device=cuda)
     out = torch.full((n,), 0.75, device=cuda)
-    call("ngs_eval_field_binned", Grid(), None, ptr(cell), ptr(basis), ptr(order), n, 1.0, ptr(out), stream())
+    call("ngs_eval_field_binned", Grid(), ptr(q), ptr(cell), ptr(basis), ptr(order), n, 1.0, ptr(out), stream())
     assert bool((out == 0.75).all())
     # no member receives anything: a null output is not written
     call("ngs_basis_splat", Grid(), ptr(out), ptr(q), n, 1.0, 1.0, None, stream())
