@@ -958,42 +958,37 @@ static int pcg_blocks(int64_t M, int64_t* chunk) {
 
 static size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 
-static int pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, bool wide = false) {
+// Places a system's state in the workspace `ws` and returns the bytes it takes (ws null: the bytes only).
+// They never fall as M grows (the wide product's partials stay reserved above WIDE_ROWS), so a workspace
+// made for a system serves every smaller one.
+static int64_t pcg_layout(int64_t M, PcgArgs* A, char* ws, void** tab = nullptr, bool wide = false) {
     int64_t chunk;
-    int nb = pcg_blocks(M, &chunk);
-    size_t off = 0;
-    A->st = reinterpret_cast<PcgState*>(ws + off);
-    off += al256(sizeof(PcgState));
-    A->partials = reinterpret_cast<double*>(ws + off);
-    off += al256(sizeof(double) * 3 * nb);
-    A->pq = A->partials;
-    A->npq = nb;
-    if (M <= WIDE_ROWS) {
-        if (wide) {
-            A->pq = reinterpret_cast<double*>(ws + off);
-            A->npq = 2 * nb;
-        }
-        off += al256(sizeof(double) * 2 * nb);
-    }
-    A->r = reinterpret_cast<float*>(ws + off);
-    off += al256(sizeof(float) * M);
-    A->p = reinterpret_cast<float*>(ws + off);
-    off += al256(sizeof(float) * M);
-    A->q = reinterpret_cast<float*>(ws + off);
-    off += al256(sizeof(float) * M);
-    if (tab) *tab = ws + off;
+    const int nb = pcg_blocks(M, &chunk);
+    int64_t off = 0;
+    auto take = [&](size_t bytes) {
+        char* p = ws ? ws + off : nullptr;
+        off += (int64_t)al256(bytes);
+        return p;
+    };
+    A->st = reinterpret_cast<PcgState*>(take(sizeof(PcgState)));
+    A->partials = reinterpret_cast<double*>(take(sizeof(double) * 3 * nb));
+    double* wide_pq = reinterpret_cast<double*>(take(sizeof(double) * 2 * std::min<int64_t>(nb, WIDE_ROWS / 256)));
+    A->pq = wide ? wide_pq : A->partials;
+    A->npq = wide ? 2 * nb : nb;
+    A->r = reinterpret_cast<float*>(take(sizeof(float) * M));
+    A->p = reinterpret_cast<float*>(take(sizeof(float) * M));
+    A->q = reinterpret_cast<float*>(take(sizeof(float) * M));
+    char* entry = take(512);
+    if (tab) *tab = entry;
     A->nblocks = nb;
     A->chunk = chunk;
     A->M = M;
-    return (int)0;
+    return off;
 }
 
 static int64_t pcg_ws_bytes(int64_t M) {
-    int64_t chunk;
-    int nb = pcg_blocks(M, &chunk);
-    return (int64_t)(al256(sizeof(PcgState)) + al256(sizeof(double) * 3 * nb) +
-                     (M <= WIDE_ROWS ? al256(sizeof(double) * 2 * nb) : 0) + 3 * al256(sizeof(float) * M) + 512 +
-                     al256(sizeof(int32_t) * nb));
+    PcgArgs A{};
+    return pcg_layout(M, &A, nullptr);
 }
 
 struct HostState {
@@ -1646,17 +1641,14 @@ int ngs_pcg_solve_runs_noalloc(const int32_t* runs, const float* rvals, const fl
     }
     NGS_REQUIRE(runs && rvals && inv_diag && b && x, "ngs_pcg_solve_runs_noalloc: null array");
     NGS_REQUIRE(M <= RUN_START_MASK + 1, "ngs_pcg_solve_runs_noalloc: too many rows for run words");
-    const int64_t need = pcg_ws_bytes(M);
-    if (need > (int64_t)NGS_PCG_NOALLOC_SCRATCH_BYTES) {
-        set_error("ngs_pcg_solve_runs_noalloc: " + std::to_string(M) + " rows need " + std::to_string(need) +
+    if (M > NGS_PCG_NOALLOC_MAX_ROWS) {
+        set_error("ngs_pcg_solve_runs_noalloc: " + std::to_string(M) + " rows need " + std::to_string(pcg_ws_bytes(M)) +
                   " bytes of workspace, above the " + std::to_string((int64_t)NGS_PCG_NOALLOC_SCRATCH_BYTES) +
                   "-byte scratch array (at most " + std::to_string((int64_t)NGS_PCG_NOALLOC_MAX_ROWS) +
                   " rows); use ngs_pcg_solve_runs with a workspace");
         return NGS_ERR_CAPACITY;
     }
-    // the advertised row limit is exactly the largest system whose layout fits the array
-    NGS_REQUIRE(pcg_ws_bytes(NGS_PCG_NOALLOC_MAX_ROWS) <= (int64_t)NGS_PCG_NOALLOC_SCRATCH_BYTES &&
-                    pcg_ws_bytes(NGS_PCG_NOALLOC_MAX_ROWS + 1) > (int64_t)NGS_PCG_NOALLOC_SCRATCH_BYTES,
+    NGS_REQUIRE(pcg_ws_bytes(NGS_PCG_NOALLOC_MAX_ROWS) <= (int64_t)NGS_PCG_NOALLOC_SCRATCH_BYTES,
                 "ngs_pcg_solve_runs_noalloc: row limit does not match the workspace layout");
     void* ws = nullptr;
     if (int r = scratch_address(&ws)) return r;
