@@ -26,11 +26,13 @@ import torch
 from . import _lib
 from ._lib import NgsError, call, lib, ptr, stream
 
+# Settings of the methods, as their functions below take them when called without. The iterations per launch
+# sequence of solve() are the string's, or where it names none PCG_CHUNK (FILTER_CHUNK for filtered solves).
 DEFAULTS = {"pcg": {"tol": 1e-5, "maxiter": -1, "res_fix": False, "verbose": False, "chunk": 32},
             "mixed": {"tol": 1e-2, "fast_tol": 1e-4, "fast_maxiter": 1000, "verbose": False, "chunk": 32},
             "cholmod": {"tol": 1e-6, "verbose": False, "chunk": 32},
             "refine": {"tol": 1e-8, "maxiter": 100000, "inner_tol": 1e-4, "max_outer": 20, "verbose": False,
-                       "chunk": 32}}
+                       "chunk": None}}
 
 # Iterations per launch sequence of a solver string that names no chunk. A sequence costs a
 # host read (~25 us), and the iterations left in it when the solve ends cost their empty launches (6 us each on
@@ -39,16 +41,22 @@ DEFAULTS = {"pcg": {"tol": 1e-5, "maxiter": -1, "res_fix": False, "verbose": Fal
 PCG_CHUNK = 16
 
 
-def parse_solver(spec: str):
+def _parse(spec: str):
+    """The method and the settings that the string itself names."""
     parts = spec.split("@")
     name = parts[0]
     if name not in DEFAULTS:
         raise NotImplementedError(f"solver {name!r} (supported: {sorted(DEFAULTS)})")
-    conf = dict(DEFAULTS[name])
+    named = {}
     for p in parts[1:]:
         k, v = p.split("=", 1)
-        conf[k] = ast.literal_eval(v)
-    return name, conf
+        named[k] = ast.literal_eval(v)
+    return name, named
+
+
+def parse_solver(spec: str):
+    name, named = _parse(spec)
+    return name, {**DEFAULTS[name], **named}
 
 
 class CSRSystem:
@@ -476,8 +484,9 @@ def inner_tolerance(tol, inner_tol, outer, filtered=False):
     return inner_tol
 
 
-def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, chunk=32):
-    """FP64 iterative refinement with FP32 PCG inner solves. Returns (x64, SolveInfo)."""
+def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, chunk=None):
+    """FP64 iterative refinement with FP32 PCG inner solves; chunk None: FILTER_CHUNK for filtered ones, else
+    PCG_CHUNK. Returns (x64, SolveInfo)."""
     M = system.M
     b64 = b.double().contiguous()
     x64 = torch.zeros(M, dtype=torch.float64, device=system.device)
@@ -488,8 +497,8 @@ def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, ch
     nb = bb ** 0.5
     rel = (rr ** 0.5) / nb if nb > 0 else 0.0
     filt = system_filter(system) if rel > tol else None
-    if filt is not None:
-        chunk = min(chunk, FILTER_CHUNK)
+    if chunk is None:
+        chunk = PCG_CHUNK if filt is None else FILTER_CHUNK
     while rel > tol and info.outer < max_outer:
         e, inner = pcg(system, r64.float(), tol=inner_tolerance(tol, inner_tol, info.outer, filt is not None),
                        maxiter=maxiter, chunk=chunk, raise_on_cap=False, filt=filt)
@@ -612,8 +621,9 @@ def solve(system, b, spec: str = "pcg"):
     """Dispatch on a solver string. Returns (x, SolveInfo): x is float32, or float64 for "refine"
     (the refinement's FP64 iterate, whose residual SolveInfo.rel_resid reports) and "cholmod" (the
     FP64 direct solution)."""
-    name, conf = parse_solver(spec)
-    chunk = conf["chunk"] if "@chunk=" in spec else PCG_CHUNK
+    name, named = _parse(spec)
+    conf = {**DEFAULTS[name], **named}
+    chunk = named.get("chunk", PCG_CHUNK)
     if name == "pcg":
         x, info = pcg(system, b, tol=conf["tol"], maxiter=conf["maxiter"], chunk=chunk)
     elif name == "mixed":
@@ -625,7 +635,7 @@ def solve(system, b, spec: str = "pcg"):
         # the FP64 iterate is the solution: its FP64 residual is the one SolveInfo reports (its FP32
         # rounding would sit at the FP32 floor, ~1e-8 relative, above the tighter tolerances)
         x, info = refine(system, b, tol=conf["tol"], inner_tol=conf["inner_tol"], max_outer=conf["max_outer"],
-                         maxiter=conf["maxiter"], chunk=chunk)
+                         maxiter=conf["maxiter"], chunk=conf["chunk"])
     if conf.get("verbose"):
         print("PCG Iteration ended in", info.iters)
     return x, info
