@@ -21,7 +21,7 @@ from . import solver as _solver
 from ._lib import call, ptr, stream
 from .bases import ensure_device_tables
 from .hashtree import HashTree
-from .reconstructor import PointBinning, Reconstructor
+from .reconstructor import MeanWeight, PointBinning, Reconstructor
 
 
 class DifferentiableScreenedPoisson:
@@ -63,6 +63,7 @@ class DifferentiableScreenedPoisson:
         scale = self.split(scale_cat.double())
         n = self.xyz.shape[0]
         self.alpha = alpha
+        mean = MeanWeight(alpha)
         self.systems, self.x, self.coarse = {}, {}, {}
         self.infos = {}
         for d in range(self.L - 1, -1, -1):
@@ -77,7 +78,7 @@ class DifferentiableScreenedPoisson:
             for dd in coarser:
                 self._field_at_points(dd, self.x[dd], X)
                 call("ngs_rhs_cross_stiffness", tree.level(d), tree.level(dd), ptr(self.x[dd]), ptr(rhs), stream())
-            bins = PointBinning(tree, self.xyz, d, alpha)
+            bins = PointBinning(tree, self.xyz, d, alpha, mean=mean)
             system = self.recon.assemble_level(d, bins, X if coarser else None, sf, self.delta, rhs)
             x, info = _solver.solve(system, rhs, self.solver)
             self.systems[d] = system

@@ -11,12 +11,25 @@ from .grid import SparseGrid
 from .hashtree import HashTree
 
 
+class MeanWeight:
+    """Mean of per-point weights: summed on the device at once, read back by the first value()."""
+
+    def __init__(self, alpha):
+        self._mean = alpha.detach().mean(dtype=torch.float64) if alpha.numel() else 0.0
+
+    def value(self) -> float:
+        if isinstance(self._mean, torch.Tensor):
+            self._mean = self._mean.item()
+        return self._mean
+
+
 class PointBinning:
     """Points of the screening term binned by their containing cell at one level, with the 3x3
     per-axis basis values of the 27 voxels around each point (reconstructor.py:111-120). Per-point
     arrays are stored in bin order: slot k holds point perm[k]."""
 
-    def __init__(self, tree: HashTree, xyz, d: int, alpha, _finalize=True):
+    def __init__(self, tree: HashTree, xyz, d: int, alpha, _finalize=True, mean=None):
+        """alpha: one weight, or one per point, then with their MeanWeight where several levels share it."""
         n = xyz.shape[0]
         s = tree.strides[d]
         dev = tree.device
@@ -28,6 +41,7 @@ class PointBinning:
         self.cells = SparseGrid.for_points(qmin, qmax, s, dev)
         self.cells.mark_coords(cell)
         self._pending = (cell, b)
+        self.alpha_mean = (mean or MeanWeight(alpha)) if isinstance(alpha, torch.Tensor) else None
         if _finalize:
             self.cells.finalize(emit=False)
             self._bucket(alpha)
@@ -35,7 +49,8 @@ class PointBinning:
     @classmethod
     def levels(cls, tree: HashTree, xyz, levels, alpha):
         """{d: PointBinning} of several levels, their cell counts read in one device-to-host read."""
-        out = {d: cls(tree, xyz, d, alpha, _finalize=False) for d in levels}
+        mean = MeanWeight(alpha) if isinstance(alpha, torch.Tensor) else None
+        out = {d: cls(tree, xyz, d, alpha, _finalize=False, mean=mean) for d in levels}
         SparseGrid.finalize_all([b.cells for b in out.values()], emit=False)
         for b in out.values():
             b._bucket(alpha)
@@ -69,7 +84,7 @@ class PointBinning:
         obj.n = 0
         obj.cells = SparseGrid.empty(tree.device)
         obj.cell_start = torch.zeros(1, dtype=torch.int32, device=tree.device)
-        obj.perm = obj.b = obj.alpha = obj.point_cell = None
+        obj.perm = obj.b = obj.alpha = obj.alpha_mean = obj.point_cell = None
         obj.ncells = 0
         obj.alpha_scalar = 0.0
         return obj
@@ -249,14 +264,15 @@ class Reconstructor:
     def _screening_strength(self, d, bins, sf):
         """Mean diagonal of the screening term over that of the stiffness, from the sizes: a point adds
         alpha sf prod_axes int B^2 = alpha sf 2.2^3 to the diagonals in all, a row's stiffness is
-        3 int B'^2 (int B^2)^2 s = 58.08 s. Per-point weights stand in the middle of the filters' range
-        (their values are on the device), 0 without points."""
+        3 int B'^2 (int B^2)^2 s = 58.08 s. Per-point weights count with their mean, which is on the device: a
+        function that reads it, called by the solves that choose a filter. 0 without points."""
         if not bins.n:
             return 0.0
-        if bins.alpha is not None:
-            return 0.2
         M = self.hash_tree.level(d).M
-        return sf * bins.alpha_scalar * bins.n * 2.2 ** 3 / (M * 58.08 * self.hash_tree.strides[d])
+        unit = sf * bins.n * 2.2 ** 3 / (M * 58.08 * self.hash_tree.strides[d])
+        if bins.alpha_mean is not None:
+            return lambda mean=bins.alpha_mean: unit * mean.value()
+        return unit * bins.alpha_scalar
 
     def _add_field_at_points(self, d, sol, xyz, bins, out):
         """out += level d's field at the screening points (ngs_eval_field's values bit for bit), read

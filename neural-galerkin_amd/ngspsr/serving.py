@@ -293,8 +293,9 @@ class ReconstructionServer:
         rel = math.sqrt(rr) / nb if nb > 0 else 0.0
         info = _solver.SolveInfo()
         filt = _solver.system_filter(system) if rel > self.tol else None
+        screened = rel > self.tol and _solver.is_screened(system)
         while rel > self.tol and info.outer < 20:
-            inner_tol = _solver.inner_tolerance(self.tol, self.inner_tol, info.outer, filt is not None)
+            inner_tol = _solver.inner_tolerance(self.tol, self.inner_tol, info.outer, screened)
             e, inner = self.pool.solve(system, r64.float(), tol=inner_tol, filt=filt)
             x64 += e.double()
             info.iters += inner.iters

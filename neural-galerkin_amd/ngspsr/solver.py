@@ -154,11 +154,19 @@ class RunSystem:
         self.level_grid = None
         return self
 
-    def set_level(self, grid, stride: int, screening: float):
+    def set_level(self, grid, stride: int, screening):
         """The level's SparseGrid (rows in rank order) and stride, and the strength of its screening term
-        beside the stiffness (mean diagonal of one over the other; 0 without screening): what filter()
-        needs. Held by the system, since the filter's words are made from the grid."""
-        self.level_grid, self.level_stride, self.screening = grid, int(stride), float(screening)
+        beside the stiffness (mean diagonal of one over the other; 0 without screening; or a function
+        that returns it): what filter() needs. Held by the system, since the filter's words are made from the
+        grid."""
+        self.level_grid, self.level_stride, self.screening = grid, int(stride), screening
+
+    def screening_strength(self) -> float:
+        if self.level_grid is None:
+            return 0.0
+        if callable(self.screening):
+            self.screening = self.screening()
+        return float(self.screening)
 
     # P's weights at offsets with 1, 2, 3 non-zero components, by the screening strength up to which they
     # hold. A stiffness-dominated matrix wants faces damped less than edges and corners lifted; the more
@@ -173,7 +181,10 @@ class RunSystem:
         """The filtered preconditioner of this system for pcg (its words tensor and the kernels' struct),
         or None: unknown level, unpacked values, or no screening (there Jacobi needs as few iterations:
         32 against 38 on a 11k-row level of noisy ellipsoids)."""
-        if self._packed is None or self.level_grid is None or not self.screening > 0 or self.M == 0:
+        if self._packed is None or self.M == 0:
+            return None
+        strength = self.screening_strength()
+        if not strength > 0:
             return None
         g = self.level_grid
         lv = _lib.Level()
@@ -185,7 +196,7 @@ class RunSystem:
         call("ngs_level_filter_words", lv, ptr(words), stream())
         f = _lib.PcgFilter()
         f.words = words.data_ptr()
-        f.weights[:] = next(w for top, w in self.FILTERS if self.screening <= top)
+        f.weights[:] = next(w for top, w in self.FILTERS if strength <= top)
         return Filter(words, f)
 
     def _pack(self, rvals, layout=None):
@@ -467,21 +478,38 @@ FILTER_CHUNK = 8  # iterations per launch sequence of a filtered solve (11-25 it
 #                   Jacobi's 26-60): one host read per sequence against up to 7 empty iterations
 
 
+# Screening strength from which the refined and adjoint solves are filtered. Below it the filter saves too few
+# iterations for its step, its words and its second sequence (solve to 1e-6, us, Jacobi / filtered at strength
+# 0.0003, 0.001, 0.004, 0.016): 9.4k rows 460 598, 464 514, 462 504, 461 461; 49k rows 621 780, 643 791, 647
+# 680, 642 613; 276k rows 1259 1577, 1260 1538, 1288 1432, 1294 1141; 1.23M rows 3932 4342, 4043 4346, 4044
+# 3903, 4049 3203.
+FILTER_STRENGTH = 0.003
+
+
 def system_filter(system):
-    """The system's filtered preconditioner for the inner solves of iterative refinement, or None."""
-    return system.filter() if isinstance(system, RunSystem) else None
+    """The system's filtered preconditioner for the inner solves of iterative refinement and the adjoint, or
+    None: no form or level for one, or screening too weak for it to pay."""
+    if not isinstance(system, RunSystem) or not system.screening_strength() >= FILTER_STRENGTH:
+        return None
+    return system.filter()
 
 
-def inner_tolerance(tol, inner_tol, outer, filtered=False):
+def inner_tolerance(tol, inner_tol, outer, screened=False):
     """Relative tolerance of an inner FP32 solve of iterative refinement. Targets the FP32 solver
     reaches on its own (tol >= 1e-6) are aimed at directly by the first inner solve, to half the
     target so that its FP32 rounding still lands below it, and verified in FP64: one FP32 solve and
-    one FP64 residual. Tighter targets take inner_tol per step (each step gains that factor). A filtered
-    solve gains nearly a factor of two per iteration: it goes to 0.3 of the target, so that where it stops
-    inside that last factor leaves no larger an error than Jacobi's smaller steps did."""
+    one FP64 residual. Tighter targets take inner_tol per step (each step gains that factor). Screened
+    systems (those that can be filtered) go to 0.3 of the target: a filtered solve gains nearly a factor of
+    two per iteration, and where it stops inside that last factor is to leave no larger an error than
+    Jacobi's smaller steps; Jacobi on the weakly screened ones costs one iteration more for it."""
     if outer == 0 and tol >= FP32_REACH:
-        return (0.3 if filtered else 0.5) * tol
+        return (0.3 if screened else 0.5) * tol
     return inner_tol
+
+
+def is_screened(system):
+    """Whether system_filter chooses for this system by its screening strength."""
+    return isinstance(system, RunSystem) and system.is_packed and system.screening_strength() > 0
 
 
 def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, chunk=None):
@@ -497,10 +525,11 @@ def refine(system, b, tol=1e-8, inner_tol=1e-4, max_outer=20, maxiter=100000, ch
     nb = bb ** 0.5
     rel = (rr ** 0.5) / nb if nb > 0 else 0.0
     filt = system_filter(system) if rel > tol else None
+    screened = rel > tol and is_screened(system)
     if chunk is None:
         chunk = PCG_CHUNK if filt is None else FILTER_CHUNK
     while rel > tol and info.outer < max_outer:
-        e, inner = pcg(system, r64.float(), tol=inner_tolerance(tol, inner_tol, info.outer, filt is not None),
+        e, inner = pcg(system, r64.float(), tol=inner_tolerance(tol, inner_tol, info.outer, screened),
                        maxiter=maxiter, chunk=chunk, raise_on_cap=False, filt=filt)
         x64 += e.double()
         info.iters += inner.iters
