@@ -352,6 +352,10 @@ int ngs_stencil_residual_f64(ngs_stencil op, const double *b, const double *x, d
  * out[i] += scale * sum_p w[p] B_i(p) over the 27 voxels of g around every point. */
 int ngs_basis_splat(ngs_grid g, const float *w, const float *xyz, int64_t n, float inv_voxel_size, double scale,
                     double *out, ngs_stream_t s);
+/* The same onto a level: its voxel count M is known before the launch, which then reserves no memory for sums
+ * that a large level does not take (faster from about 1e5 points on). */
+int ngs_basis_splat_level(ngs_level level, const float *w, const float *xyz, int64_t n, float inv_voxel_size,
+                          double scale, double *out, ngs_stream_t s);
 /* Transpose of the cross-level stiffness of ngs_rhs_cross_stiffness:
  * out_coarse[j] += scale * sum_i K_{d,dd}(i, j) g_fine[i]. The backward of the cascadic RHS
  * correction (reconstructor.py:153-168) through Solver.backward (solver.py:91-98). */

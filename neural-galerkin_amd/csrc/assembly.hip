@@ -609,21 +609,26 @@ __global__ void rhs_normals_gather_kernel(ngs_level tgt, ngs_level dat, const fl
 
 // FP64 sums into a grid's members from many threads. On a coarse grid a few hundred members receive
 // everything and device-scope atomics on one address take turns at the memory side (270k additions into 110
-// members: 143 us, 13 us with the LDS sums), so a block first sums into LDS and adds each of its members once, where the grid fits
-// and that is fewer global atomics than adding directly: `adds` of the whole launch against one per member
-// and block. add() and flush() are called by every thread of the block, flush() once.
+// members: 143 us, 13 us with the LDS sums), so a block first sums into LDS and adds each of its members once,
+// where the grid fits and that is fewer global atomics than adding directly: `adds` of the whole launch against
+// one per member and block, in the first `local_blocks` blocks (the flushes are what limits them). The others
+// return at once: only a launch that adds directly uses them. add() and flush() are called by every thread of
+// the block, flush() once.
 constexpr int MEMBER_LDS = 6144;  // 48 KB
 
 struct MemberSums {
     double* lds;
     double* out;
     int count;
+    unsigned blocks;  // that share the work
     bool local;
-    __device__ __forceinline__ MemberSums(const ngs_grid& g, double* out_, double* lds_, double adds)
+    __device__ __forceinline__ MemberSums(const ngs_grid& g, double* out_, double* lds_, int lds_members, double adds,
+                                          unsigned local_blocks)
         : lds(lds_), out(out_) {
         count = grid_count(g);
-        local = count <= MEMBER_LDS && 2.0 * count * gridDim.x < adds;  // uniform over the grid
-        if (local) {
+        local = count <= lds_members && 2.0 * count * local_blocks < adds;  // uniform over the grid
+        blocks = local ? local_blocks : gridDim.x;
+        if (local && blockIdx.x < blocks) {
             for (int k = threadIdx.x; k < count; k += blockDim.x) lds[k] = 0.0;
             __syncthreads();
         }
@@ -640,19 +645,58 @@ struct MemberSums {
     }
 };
 
-// Blocks for `items` work items of MemberSums kernels: 4 per thread, at most one block per CU.
-static unsigned member_blocks(int64_t items) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, items / 1024)); }
+// Launch shape of the MemberSums kernels for n points (or voxels) of `columns` bitmap columns each. Summing in
+// LDS: 4 columns per thread, at most one block per CU. Adding directly: one thread per column while a thread per
+// point would leave the chip idle, above that one per point, whose lanes add to the same members together.
+// Directly with a thread per column / per point, us: splat of 16k points on 9.6k members 28 / 30, of 30k 55 / 50,
+// of 300k on 11k and 862k members 634 / 470 and 334 / 315; transposed stiffness of 9.6k voxels 80 / 83, of 42k
+// 121 / 96, of 862k 1635 / 1097.
+constexpr int64_t MEMBER_WIDE = 24576;
+
+struct MemberGrid {
+    unsigned local_blocks, blocks;
+    int lds_members;
+    bool wide;  // a thread per column
+    // members: their number, or a bound of it. Above what LDS holds the launch reserves none, which would only
+    // lower its occupancy (3 blocks per CU: 300k points on 50k members 389 -> 419 us).
+    MemberGrid(int64_t n, int columns, int64_t members, bool bound) {
+        lds_members = (int)(members <= MEMBER_LDS ? members : bound ? MEMBER_LDS : 0);
+        const int64_t items = columns * n;
+        local_blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, items / 1024));
+        wide = n <= MEMBER_WIDE;
+        blocks = (unsigned)std::max<int64_t>(local_blocks, ((wide ? items : n) + 255) / 256);
+    }
+};
 
 // Transpose of the field evaluation: out[i] += scale * sum_p w_p B_i(p) over the 27 voxels of g
-// around each point (the adjoint of hashtree.py:157-192). One item per (point, bitmap column).
+// around each point (the adjoint of hashtree.py:157-192).
 __global__ void __launch_bounds__(256) basis_splat_kernel(ngs_grid g, const float* __restrict__ w,
                                                           const float* __restrict__ xyz, int64_t n, float inv_vs,
-                                                          double scale, double* __restrict__ out) {
-    __shared__ double lds[MEMBER_LDS];
-    const MemberSums sums(g, out, lds, 27.0 * n);
+                                                          double scale, double* __restrict__ out,
+                                                          int lds_members, unsigned local_blocks, bool wide) {
+    extern __shared__ double member_sums[];
+    const MemberSums sums(g, out, member_sums, lds_members, 27.0 * n, local_blocks);
+    if (blockIdx.x >= sums.blocks) return;
     const int s = 1 << g.log2_stride, l2 = g.log2_stride;
     const float inv_s = 1.0f / (float)s;
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 9 * n; t += (int64_t)gridDim.x * 256) {
+    if (!sums.local && !wide) {
+        const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (i >= n) return;
+        const float wi = w[i];
+        if (wi == 0.f) return;
+        int cell[3];
+        float b[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) axis_basis(xyz[3 * i + a] * inv_vs, s, inv_s, &cell[a], b[a]);
+        for (int kx = 0; kx < 3; ++kx)
+            for (int ky = 0; ky < 3; ++ky)
+                for (int kz = 0; kz < 3; ++kz) {
+                    const int id = grid_find(g, cell[0] + (kx - 1) * s, cell[1] + (ky - 1) * s, cell[2] + (kz - 1) * s);
+                    if (id >= 0) sums.add(id, scale * (double)(wi * (b[0][kx] * b[1][ky] * b[2][kz])));
+                }
+        return;
+    }
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 9 * n; t += (int64_t)sums.blocks * 256) {
         const int64_t i = t / 9;
         const int col = (int)(t - 9 * i), kx = col / 3, ky = col % 3;
         const float wi = w[i];
@@ -673,21 +717,24 @@ __global__ void __launch_bounds__(256) basis_splat_kernel(ngs_grid g, const floa
     sums.flush();
 }
 
-// Transpose of the cross-level stiffness: out_c[j] += scale * sum_i K_{d,dd}(i, j) g_f[i]. One item per (fine
-// voxel, coarse bitmap column).
+// Transpose of the cross-level stiffness: out_c[j] += scale * sum_i K_{d,dd}(i, j) g_f[i].
 __global__ void __launch_bounds__(256) cross_stiffness_t_kernel(ngs_level fine, ngs_level coarse,
                                                                 const float* __restrict__ gf, Tables T, double scale,
-                                                                double* __restrict__ out) {
-    __shared__ double lds[MEMBER_LDS];
-    const MemberSums sums(coarse.grid, out, lds, 60.0 * fine.M);
+                                                                double* __restrict__ out, int lds_members,
+                                                                unsigned local_blocks, bool wide) {
+    extern __shared__ double member_sums[];
+    const MemberSums sums(coarse.grid, out, member_sums, lds_members, 60.0 * fine.M, local_blocks);
+    if (blockIdx.x >= sums.blocks) return;
     const int sf_ = fine.stride, sc = coarse.stride, m = T.m;
     const int nrow = 3 * m + 2;
     const float fs = (float)sf_, inv_sc = 1.0f / (float)sc;
     const ngs_grid& g = coarse.grid;
     const int l2 = g.log2_stride;
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < 25 * fine.M; t += (int64_t)gridDim.x * 256) {
-        const int64_t i = t / 25;
-        const int col = (int)(t - 25 * i), kx = col / 5 - 2, ky = col % 5 - 2;
+    const bool rows = !sums.local && !wide;  // a thread per fine voxel, else one per (fine voxel, coarse column)
+    const int64_t items = rows ? fine.M : 25 * fine.M;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < items; t += (int64_t)sums.blocks * 256) {
+        const int64_t i = rows ? t : t / 25;
+        const int c0_ = rows ? 0 : (int)(t - 25 * i), c1_ = rows ? 25 : c0_ + 1;
         const float gi = gf[i];
         if (gi == 0.f) continue;
         int c[3], Q[3];
@@ -698,22 +745,25 @@ __global__ void __launch_bounds__(256) cross_stiffness_t_kernel(ngs_level fine, 
             int q = num >= 0 ? num / den : -((-num + den - 1) / den);
             Q[a] = q * sc;
         }
-        const int ix = kx * m + (Q[0] - c[0]) / sf_ + 2 * m, iy = ky * m + (Q[1] - c[1]) / sf_ + 2 * m;
-        if (ix < 0 || ix >= nrow || iy < 0 || iy >= nrow) continue;
-        int32_t id = 0;
-        const uint32_t mask = grid_column(g, (Q[0] >> l2) - g.origin[0] + kx, (Q[1] >> l2) - g.origin[1] + ky,
-                                          (Q[2] >> l2) - g.origin[2] - 2, 5, &id);
-        if (!mask) continue;
-        const float c0 = T.F[ix] * fs, c1 = T.F[iy] * fs, g0 = T.G[ix] * inv_sc, g1 = T.G[iy] * inv_sc;
+        for (int col = c0_; col < c1_; ++col) {
+            const int kx = col / 5 - 2, ky = col % 5 - 2;
+            const int ix = kx * m + (Q[0] - c[0]) / sf_ + 2 * m, iy = ky * m + (Q[1] - c[1]) / sf_ + 2 * m;
+            if (ix < 0 || ix >= nrow || iy < 0 || iy >= nrow) continue;
+            int32_t id = 0;
+            const uint32_t mask = grid_column(g, (Q[0] >> l2) - g.origin[0] + kx, (Q[1] >> l2) - g.origin[1] + ky,
+                                              (Q[2] >> l2) - g.origin[2] - 2, 5, &id);
+            if (!mask) continue;
+            const float c0 = T.F[ix] * fs, c1 = T.F[iy] * fs, g0 = T.G[ix] * inv_sc, g1 = T.G[iy] * inv_sc;
 #pragma unroll
-        for (int kz = -2; kz <= 2; ++kz) {
-            if (!((mask >> (kz + 2)) & 1u)) continue;
-            const int j = id++;
-            const int iz = kz * m + (Q[2] - c[2]) / sf_ + 2 * m;
-            if (iz < 0 || iz >= nrow) continue;
-            const float c2 = T.F[iz] * fs, g2 = T.G[iz] * inv_sc;
-            const float K = g0 * c1 * c2 + c0 * g1 * c2 + c0 * c1 * g2;
-            sums.add(j, scale * (double)(K * gi));
+            for (int kz = -2; kz <= 2; ++kz) {
+                if (!((mask >> (kz + 2)) & 1u)) continue;
+                const int j = id++;
+                const int iz = kz * m + (Q[2] - c[2]) / sf_ + 2 * m;
+                if (iz < 0 || iz >= nrow) continue;
+                const float c2 = T.F[iz] * fs, g2 = T.G[iz] * inv_sc;
+                const float K = g0 * c1 * c2 + c0 * g1 * c2 + c0 * c1 * g2;
+                sums.add(j, scale * (double)(K * gi));
+            }
         }
     }
     sums.flush();
@@ -935,12 +985,24 @@ int ngs_rhs_normals(ngs_level target, ngs_level data, const float* normals, doub
     return NGS_OK;
 }
 
+static int basis_splat(ngs_grid g, const MemberGrid& mg, const float* w, const float* xyz, int64_t n,
+                       float inv_voxel_size, double scale, double* out, ngs_stream_t s) {
+    basis_splat_kernel<<<mg.blocks, 256, sizeof(double) * mg.lds_members, S(s)>>>(
+        g, w, xyz, n, inv_voxel_size, scale, out, mg.lds_members, mg.local_blocks, mg.wide);
+    NGS_CHECK_LAUNCH();
+    return NGS_OK;
+}
+
 int ngs_basis_splat(ngs_grid g, const float* w, const float* xyz, int64_t n, float inv_voxel_size, double scale, double* out,
                     ngs_stream_t s) {
     if (n <= 0) return NGS_OK;
-    basis_splat_kernel<<<member_blocks(9 * n), 256, 0, S(s)>>>(g, w, xyz, n, inv_voxel_size, scale, out);
-    NGS_CHECK_LAUNCH();
-    return NGS_OK;
+    return basis_splat(g, MemberGrid(n, 9, 32 * g.nwords, true), w, xyz, n, inv_voxel_size, scale, out, s);
+}
+
+int ngs_basis_splat_level(ngs_level lv, const float* w, const float* xyz, int64_t n, float inv_voxel_size, double scale,
+                          double* out, ngs_stream_t s) {
+    if (n <= 0 || lv.M <= 0) return NGS_OK;
+    return basis_splat(lv.grid, MemberGrid(n, 9, lv.M, false), w, xyz, n, inv_voxel_size, scale, out, s);
 }
 
 int ngs_cross_stiffness_transpose(ngs_level fine, ngs_level coarse, const float* g_fine, double scale, double* out_coarse,
@@ -949,7 +1011,9 @@ int ngs_cross_stiffness_transpose(ngs_level fine, ngs_level coarse, const float*
     NGS_REQUIRE(coarse.stride > fine.stride, "ngs_cross_stiffness_transpose: coarse stride must exceed fine stride");
     Tables T;
     NGS_REQUIRE(tables_for(coarse.stride / fine.stride, &T), "ngs_cross_stiffness_transpose: table multiple unavailable");
-    cross_stiffness_t_kernel<<<member_blocks(25 * fine.M), 256, 0, S(s)>>>(fine, coarse, g_fine, T, scale, out_coarse);
+    const MemberGrid mg(fine.M, 25, coarse.M, false);
+    cross_stiffness_t_kernel<<<mg.blocks, 256, sizeof(double) * mg.lds_members, S(s)>>>(
+        fine, coarse, g_fine, T, scale, out_coarse, mg.lds_members, mg.local_blocks, mg.wide);
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }

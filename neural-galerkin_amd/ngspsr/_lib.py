@@ -117,6 +117,7 @@ _SIGNATURES = {
     "ngs_rhs_cross_stiffness": ([Level, Level, P, P, P], c_int32),
     "ngs_rhs_normals": ([Level, Level, P, P, P], c_int32),
     "ngs_basis_splat": ([Grid, P, P, c_int64, c_float, c_double, P, P], c_int32),
+    "ngs_basis_splat_level": ([Level, P, P, c_int64, c_float, c_double, P, P], c_int32),
     "ngs_cross_stiffness_transpose": ([Level, Level, P, c_double, P, P], c_int32),
     "ngs_pcg_workspace_bytes": ([c_int64], c_int64),
     "ngs_pcg_config": ([c_int32, c_int32, c_int32, c_int32], c_int32),

@@ -114,7 +114,7 @@ class DifferentiableScreenedPoisson:
                     continue
                 call("ngs_cross_stiffness_transpose", tree.level(d), tree.level(dd), ptr(g_b), -1.0, ptr(g_x[dd]),
                      stream())
-                call("ngs_basis_splat", tree.grids[dd].struct(), ptr(w), ptr(self.xyz), n, tree.inv_vs, -sf,
+                call("ngs_basis_splat_level", tree.level(dd), ptr(w), ptr(self.xyz), n, tree.inv_vs, -sf,
                      ptr(g_x[dd]), stream())
         return g_alpha, torch.cat([g_scale[d] for d in range(self.L)])
 
@@ -135,7 +135,7 @@ class DifferentiableScreenedPoisson:
         for d in range(self.L):
             o = torch.zeros(self.sizes[d], dtype=torch.float64, device=self.tree.device)
             if self.sizes[d]:
-                call("ngs_basis_splat", self.tree.grids[d].struct(), ptr(g), ptr(q), q.shape[0], self.tree.inv_vs, 1.0,
+                call("ngs_basis_splat_level", self.tree.level(d), ptr(g), ptr(q), q.shape[0], self.tree.inv_vs, 1.0,
                      ptr(o), stream())
             outs.append(o)
         return torch.cat(outs)
