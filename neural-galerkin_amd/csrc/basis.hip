@@ -76,6 +76,7 @@ __global__ void ddi_backward_kernel(const float* __restrict__ s, const float* __
 // the tables once). Same products and summation order as above, so the results are identical.
 constexpr int DDI_MAXC = 16;
 constexpr int DDI_LDS_BYTES = 64 * 1024;
+constexpr int LDS_PER_CU = 160 * 1024;
 
 __device__ __forceinline__ void ddi_stage_tables(const float* __restrict__ ff, const float* __restrict__ dd, int nc,
                                                  int L, float2* tab) {
@@ -130,10 +131,10 @@ __global__ void __launch_bounds__(256) ddi_forward_lds_kernel(const float* __res
 // coefficients they replace. One thread per (pair, axis) k = 3 pair + axis: the offsets, the incoming
 // gradients and the forward's results are then contiguous over the lanes too, and the 2 NC coefficients
 // of an axis fit in registers, with every loop over them unrolled. 64 pairs are 192 threads and
-// 1536 NC bytes of LDS beside the tables, so at 7 components the wave slots limit the residency, not the
-// LDS. Arithmetic and
-// summation order are those of the kernels above. 2M pairs of 7 components, forward and backward: 249 and
-// 975 us with a thread per pair (the forward's rows staged, the backward's not), 103 and 143 us in tiles.
+// 1536 NC bytes of LDS beside the tables, so at 7 components and short tables the wave slots limit the
+// residency, not the LDS. Arithmetic and summation order are those of the kernels above. 2M pairs of 7
+// components, forward and backward: 249 and 975 us with a thread per pair (the forward's rows staged, the
+// backward's not), 103 and 143 us in tiles.
 constexpr int DDI_PAIRS = 64;
 constexpr int DDI_THREADS = 3 * DDI_PAIRS;
 
@@ -289,9 +290,14 @@ static bool ddi_tile_launch(const float* s, const float* t, const int64_t* rel, 
         // every tile starts at a multiple of 64 rows, so the arrays' own alignment is the rows'
         uintptr_t al = reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(t);
         if (BWD) al |= reinterpret_cast<uintptr_t>(o1) | reinterpret_cast<uintptr_t>(o2);
-        // resident blocks: 10 of 3 waves per CU (32 wave slots), 8 tiles or fewer each before more are added
+        // Four rounds of resident blocks (10 of 3 waves per CU by the wave slots), which evens out their ends. Where
+        // the tables outweigh a tile's rows, one round of what LDS holds: every block loads the tables. Four
+        // rounds / one, us, forward: 10 components, tables of 50, 100k pairs 35.4 / 23.0 (tables only in LDS
+        // 30.8), 1M 263 / 158 (257); 7 of 50, 1M 87.8 / 63.4; but 16 of 14 478 / 502, 7 of 14 42.8 / 49.4.
         const int64_t tiles = (n + DDI_PAIRS - 1) / DDI_PAIRS;
-        const unsigned grid = (unsigned)std::min<int64_t>(tiles, 256 * 10 * 4);
+        const int64_t rows = 2LL * DDI_PAIRS * 3 * nc * 4;
+        const int64_t blocks = 4 * (bytes - rows) > 5 * rows ? 256 * std::min<int64_t>(10, LDS_PER_CU / bytes) : 256 * 10 * 4;
+        const unsigned grid = (unsigned)std::min<int64_t>(tiles, blocks);
         ddi_tile_kernel<NC, BWD><<<grid, DDI_THREADS, (size_t)bytes, st>>>(s, t, rel, n, ff, dd, L, al % 16 == 0, gp,
                                                                            gq, o1, o2);
         return true;
