@@ -598,7 +598,7 @@ __global__ void splat_bins_kernel(const uint32_t* __restrict__ ks, const int32_t
 // point of them; the FP64 sums of the lanes are then added pairwise. One lane per node waits through its 8
 // bins in a row: right where the nodes fill the chip by themselves and most bins are empty or nearly so,
 // but on grids coarse against the points (the density grid, the coarse levels) there are too few nodes to
-// hide it. Measured, us for 1 / 4 / 16 / 64 lanes:
+// hide it (gather_lanes). The kernel alone, us for 1 / 4 / 16 / 64 lanes:
 //   16.1M nodes, 2.9M points: 934 1192 3472 -     821k nodes, 270k points: 74 77 149 498
 //   220k nodes, 2M points: 348 206 136 142        51k nodes, 300k points: 214 77 34 31
 //   10k nodes, 9k points on one side: 391 137 45 14        6.2k nodes, 100k points: 535 149 40 14
@@ -1208,6 +1208,22 @@ int ngs_splat(ngs_grid g, const float* xyz, int64_t n, float inv_voxel_size, con
     return NGS_OK;
 }
 
+// Lanes per node of splat_gather_kernel: several where the nodes alone leave the chip idle, or where their bins
+// are long. The whole call with 1 / 4 / 16 / 64 lanes, us, for full boxes of nodes, 3 components:
+//   11k nodes, 0.1 points per node 42 30 30 31, 2 per node 110 63 52 55     27k, 0.1 44 32 31 41, 2 109 69 60 69
+//   64k, 0.1 52 42 46 66, 0.5 75 57 59 86, 2 120 88 86 110                  141k, 0.1 57 49 61 104, 10 443 404 279 315
+//   287k, 0.01 41 40 58 137, 0.5 117 107 126 255, 2 213 195 212 335, 10 869 694 470 541
+//   422k, 0.1 77 78 117 242, 2 252 240 266 448                              729k, 0.1 107 112 186 422, 2 354 340 393 708
+//   1.4M, 0.01 82 100 199 603, 0.5 270 284 397 1034, 2 567 569 688 1333
+// and on levels of noisy surfaces (most nodes without points): 160k nodes, 300k points 156 140 148 216; 202k, 300k 198
+// 171 172 249; 220k, 1M 424 325 290 337; 819k, 300k 200 200 267 614; 1.03M, 1M 342 336 401 -; 1.13M, 2M 442 436 498 -.
+static int gather_lanes(int64_t count, int64_t n) {
+    if (count <= 12000) return 64;
+    if (count <= 100000 || (count <= 400000 && n >= 4 * count)) return 16;
+    if (count <= 400000 || (count <= 1500000 && 4 * n >= 3 * count)) return 4;
+    return 1;
+}
+
 static int splat_gather_layout(int64_t n, int64_t count, size_t* tmp, size_t off[8], size_t* total) {
     auto al = [](size_t x) { return (x + 255) / 256 * 256; };
     const int bits = 32 - __builtin_clz((uint32_t)count);  // the keys run up to count
@@ -1270,16 +1286,17 @@ int ngs_splat_gather(ngs_grid g, const int32_t* node_coords, int64_t count, cons
     splat_bins_kernel<<<grid1d(n, 256), 256, 0, st>>>(ks, order, n, (uint32_t)count, xyz, data, ncomp, scale, bstart,
                                                       bend, bxyz, brow);
     NGS_CHECK_LAUNCH();
-    // lanes per node: enough threads for the chip (500k resident), see the kernel's figures
     auto gather = [&](auto lanes) {
         constexpr int G = decltype(lanes)::value;
         splat_gather_kernel<G><<<grid1d(count, 256 / G), 256, 0, st>>>(
             g, node_coords, count, inv_voxel_size, data ? ncomp : 0, bstart, bend, bxyz, brow, post, acc);
     };
-    if (count > 1500000) gather(std::integral_constant<int, 1>());
-    else if (count > 400000) gather(std::integral_constant<int, 4>());
-    else if (count > 12000) gather(std::integral_constant<int, 16>());
-    else gather(std::integral_constant<int, 64>());
+    switch (gather_lanes(count, n)) {
+        case 1: gather(std::integral_constant<int, 1>()); break;
+        case 4: gather(std::integral_constant<int, 4>()); break;
+        case 16: gather(std::integral_constant<int, 16>()); break;
+        default: gather(std::integral_constant<int, 64>());
+    }
     NGS_CHECK_LAUNCH();
     return NGS_OK;
 }

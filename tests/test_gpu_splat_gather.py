@@ -70,7 +70,7 @@ def test_splat_gather_density_all_points():
 
 def test_splat_gather_duplicated_cloud():
     """A cloud where most points repeat a few positions: the nodes around those positions gather
-    long bins (one thread walks all of their points), and the sums still equal the scatter's."""
+    long bins (a few lanes walk all of their points), and the sums still equal the scatter's."""
     from ngspsr._lib import call, lib, ptr, stream
     from ngspsr.grid import SparseGrid
     n = 40000
