@@ -1009,9 +1009,14 @@ static HostState& host_state() {
 enum : int32_t { SYS_CSR = 0, SYS_STENCIL = 1, SYS_RUNS = 2, SYS_PACKED = 3 };
 
 // Flags of a launch sequence (which kernels the table's systems need).
-enum : int32_t { FLAG_STENCIL = 1, FLAG_RUNS = 2, FLAG_NO_CSR = 4, FLAG_PACKED = 8, FLAG_FILTER = 16,
-// one packed system of at most WIDE_ROWS rows laid out for the wide product (internal)
-                 FLAG_WIDE = 32 };
+enum : int32_t {
+    FLAG_STENCIL = 1,
+    FLAG_RUNS = 2,
+    FLAG_NO_CSR = 4,
+    FLAG_PACKED = 8,
+    FLAG_FILTER = 16,
+    FLAG_WIDE = 32,  // internal: one packed system of at most WIDE_ROWS rows, laid out for the wide product
+};
 
 struct BatchSys {
     PcgArgs a;
